@@ -743,21 +743,33 @@ static unsigned march_grid(const Level& lv, int d, int sl, bool fused) {
 
 // One directional flux pass (not fused) with face values of type R.
 extern "C++" {
+template <typename R, bool RW, int LN>
+static void launch_solid_x(tj_ctx* c, const MF& Uin, const FacesT<R>& F, long long waves) {
+    hipLaunchKernelGGL((k_flux_x_s<2, LN, RW, R>), dim3(grid1(waves, 4)), dim3(256), 0, c->stream, c->lv, Uin, F, c->d_clk);
+}
+template <typename R, bool RW, int D>
+static void launch_solid_yz(tj_ctx* c, const MF& Uin, const FacesT<R>& F) {
+    using T = STile<2, R>;
+    const Level& lv = c->lv;
+    const unsigned g = grid1(lv.n[0], T::TC) * grid1(lv.n[D] + 1, T::PER) * (unsigned)lv.n[D == 1 ? 2 : 1];
+    hipLaunchKernelGGL((k_flux_yz_s<2, D, RW, R>), dim3(g), dim3(256), 0, c->stream, lv, Uin, F, c->d_clk);
+}
 template <typename R, bool RW>
 static void launch_pass_solid(tj_ctx* c, const MF& Uin, int d, const FacesT<R>* F) {
-    const Level& lv = c->lv;
     if (d == 0) {
-        const long long nseg = (lv.n[0] + 1 + 62) / 63;
-        const unsigned g = grid1(nseg * lv.n[1] * lv.n[2], 4);
-        hipLaunchKernelGGL((k_flux_x_s<2, RW, R>), dim3(g), dim3(256), 0, c->stream, lv, Uin, F[0], c->d_clk);
+        // segments of 64 or 32 lanes along x, whichever needs fewer waves: a
+        // segment spends one lane on its neighbour's face state, and its last
+        // one the lanes past the row's end (145 faces: 3 x 64 or 5 x 32 lanes)
+        const Level& lv = c->lv;
+        const long long rows = (long long)lv.n[1] * lv.n[2];
+        const long long w64 = (long long)grid1(lv.n[0] + 1, 63) * rows;
+        const long long w32 = (long long)grid1(lv.n[0] + 1, 31) * ((rows + 1) / 2);
+        if (w32 < w64) launch_solid_x<R, RW, 32>(c, Uin, F[0], w32);
+        else launch_solid_x<R, RW, 64>(c, Uin, F[0], w64);
     } else if (d == 1) {
-        const int sl = seg_for(c, TJ_KPTR(k_flux_lmarch_s<2, 1, RW, R>), 1, false);
-        hipLaunchKernelGGL((k_flux_lmarch_s<2, 1, RW, R>), dim3(march_grid(lv, 1, sl, false)), dim3(256), 0, c->stream,
-                           lv, Uin, F[1], sl, c->d_clk);
+        launch_solid_yz<R, RW, 1>(c, Uin, F[1]);
     } else {
-        const int sl = seg_for(c, TJ_KPTR(k_flux_lmarch_s<2, 2, RW, R>), 2, false);
-        hipLaunchKernelGGL((k_flux_lmarch_s<2, 2, RW, R>), dim3(march_grid(lv, 2, sl, false)), dim3(256), 0, c->stream,
-                           lv, Uin, F[2], sl, c->d_clk);
+        launch_solid_yz<R, RW, 2>(c, Uin, F[2]);
     }
 }
 template <typename R, bool MX>

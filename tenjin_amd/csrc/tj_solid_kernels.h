@@ -59,197 +59,210 @@ __device__ __forceinline__ SSt<NM, R> state_dn(const SSt<NM, R>& S) {
 template <int NM, typename R>
 __device__ __forceinline__ void flip_s(SSt<NM, R>& S, int d) { S.u[d] = -S.u[d]; }
 
-// x pass of the solid path (same wave layout as k_flux_x, no THINC).
-template <int NM, bool RW, typename R>
+// Flux passes of the solid path, one reconstruction per cell: a lane
+// reconstructs one cell (MUSCL, then p2c + sound speed of both face states)
+// and face f takes its left state UR(f-1) from lane - 1, the cell one below
+// along D, so a segment of LN lanes gives LN - 1 faces.  The domain's end
+// faces take the image of the edge cell's own state.
+//
+// Bound by VALU issue: some 3500 instructions a face in FP64 (two waves per
+// SIMD), 1900 in FP32 (four).  A march of one wave along D, with the rows in
+// registers, keeps one wave per SIMD in flight and gives a small level few
+// waves: y and z passes of 144^3 in FP64 780 us against 490 here (512^2: 102
+// against 54), of 203 x 160 x 131 in FP32 430 against 285.  Blocks run in XCD
+// order: tiles side by side share the cache lines of rows whose pitch is no
+// multiple of the line (the same FP32 y pass 395 us in round-robin order).
+// The face of a lane: c its lower face along D, PL / PR the reconstructed
+// primitives of its cell, LN lanes to a segment (ld the lane within it).
+// The right state moves up before the left one is built, so two face states
+// are live at a time.
+template <int NM, int D, bool RW, typename R>
+__device__ __forceinline__ void face_s(const Level& lv, const SPrim<NM, R>& PL, const SPrim<NM, R>& PR, int c, bool face,
+                                       R* Fv, unsigned& st) {
+    const int nd = lv.n[D];
+    SSt<NM, R> Lf;
+    {
+        SSt<NM, R> SRs;
+        p2c_sound_s<NM, RW, R>(lv, PR, D, SRs);
+        Lf = state_dn<NM, R>(SRs);
+        if (c == 0) {
+            Lf = SRs;
+            if (lv.bc_lo[D]) flip_s<NM, R>(Lf, D);
+        }
+    }
+    SSt<NM, R> Rf;
+    p2c_sound_s<NM, RW, R>(lv, PL, D, Rf);
+    if (c == nd && lv.bc_hi[D]) flip_s<NM, R>(Rf, D);
+    if (face) wave5<NM, RW, R>(lv, Lf, Rf, D, Fv, st);
+}
+
+// x pass: waves of 64 / LN rows by LN lanes along x (144^3 FP64: 555 us with
+// segments of 64, 467 with 32; 203 x 160 x 131 FP32: 340 and 309, and 381 with
+// 16, whose loads fall into four row pieces).
+template <int NM, int LN, bool RW, typename R>
 __global__ __launch_bounds__(256) void k_flux_x_s(Level lv, MF U, FacesT<R> F, Clock* clk) {
     if (clk->done) return;
-    constexpr int PER = 63;
+    constexpr int PER = LN - 1;
     constexpr int NF = 3 * NM + 17;
-    const int lane = threadIdx.x & 63;
-    const long long wave = (long long)blockIdx.x * (blockDim.x >> 6) + wave_in_block();
-    const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
+    const int lane = threadIdx.x & 63, ld = lane % LN;
+    const long long wave = xcd_block(blockIdx.x, gridDim.x, 2) * (blockDim.x >> 6) + wave_in_block();
+    const int nx = lv.n[0], ny = lv.n[1];
     const int nseg = (nx + 1 + PER - 1) / PER;
-    if (wave >= (long long)nseg * ny * nz) return;
+    const long long rows = (long long)ny * lv.n[2];
+    if (wave >= nseg * ((rows + 64 / LN - 1) / (64 / LN))) return;
     const int seg = (int)(wave % nseg);
-    const long long row = wave / nseg;
+    const long long row0 = wave / nseg * (64 / LN) + lane / LN;
+    const bool act = row0 < rows;
+    const long long row = act ? row0 : rows - 1;
     const int j = (int)(row % ny), k = (int)(row / ny);
-    const int c = seg * PER - 1 + lane;
+    const int c = seg * PER - 1 + ld;
     bool fl;
     const int s = bcmap(c, nx, lv.bc_lo[0], lv.bc_hi[0], fl);
-    SSt<NM, R> SLs, SRs;
+    SPrim<NM, R> PL, PR;
     {
-        SPrim<NM, R> Pm, Pc, Pp, PL, PR;
+        SPrim<NM, R> Pm, Pc, Pp;
         load_sprim<NM, R>(lv, U, s - 1, j, k, Pm);
         load_sprim<NM, R>(lv, U, s, j, k, Pc);
         load_sprim<NM, R>(lv, U, s + 1, j, k, Pp);
         muscl_s<NM, R>(Pm, Pc, Pp, PL, PR);
-        p2c_sound_s<NM, RW, R>(lv, PL, 0, SLs);
-        p2c_sound_s<NM, RW, R>(lv, PR, 0, SRs);
     }
-    SSt<NM, R> Lf = state_dn<NM, R>(SRs);
     unsigned st = 0;
-    if (lane >= 1 && c >= 0 && c <= nx) {
-        if (c == 0) {
-            Lf = SRs;
-            if (lv.bc_lo[0]) flip_s<NM, R>(Lf, 0);
-        }
-        SSt<NM, R> Rf = SLs;
-        if (c == nx && lv.bc_hi[0]) flip_s<NM, R>(Rf, 0);
-        R Fv[NF];
-        wave5<NM, RW, R>(lv, Lf, Rf, 0, Fv, st);
+    R Fv[NF];
+    const bool face = act && ld >= 1 && c >= 0 && c <= nx;
+    face_s<NM, 0, RW, R>(lv, PL, PR, c, face, Fv, st);
+    if (face) {
 #pragma unroll
         for (int q = 0; q < NF; ++q) F.at(q, c, j, k) = Fv[q];
     }
     if (st) atomicOr(&clk->status, st);
 }
 
-// A solid face state in LDS, one slot per field, lane-minor (conflict-free).
+// y / z pass: a block of four waves owns 16 columns along x by one segment of
+// 16 cells along D.  The primitives of the tile and its two halo rows are
+// staged in LDS (rows of 16 cells, coalesced); lanes then run along D, four
+// columns to a wave, and the fluxes go back through LDS to rows of 16.  Lanes
+// that load and store their own 4 x 16 tile in memory order instead, without
+// LDS, take 505 us against 490 (144^3 FP64) and 860 against 285 (FP32), whose
+// row pieces are then 32 and 16 bytes.
 template <int NM, typename R>
-struct SStSlots {
-    static constexpr int N = 5 * NM + 15;
+struct STile {
+    static constexpr int TC = 16, LN = 16;       // columns, lanes along D
+    static constexpr int PER = LN - 1;           // faces per segment
+    static constexpr int ROWS = LN + 2;          // rows c0 - 1 .. c0 + LN
+    static constexpr int NP = 3 * NM + 13;       // primitives
+    static constexpr int NF = 3 * NM + 17;       // flux components
+    static constexpr int FR = PER + 2;           // column pitch of the staged fluxes
+    static constexpr int WORDS = NP * TC * ROWS > NF * TC * FR ? NP * TC * ROWS : NF * TC * FR;
 };
-template <int NM, typename R>
-__device__ __forceinline__ void sst_store(R* sh, int lane, const SSt<NM, R>& S) {
-    int q = 0;
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        sh[(q++) * 64 + lane] = S.al[m];
-        sh[(q++) * 64 + lane] = S.ar[m];
-        sh[(q++) * 64 + lane] = S.are[m];
-    }
-    sh[(q++) * 64 + lane] = S.rho;
-    sh[(q++) * 64 + lane] = S.E;
-    sh[(q++) * 64 + lane] = S.p;
-    sh[(q++) * 64 + lane] = S.a;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        sh[(q++) * 64 + lane] = S.u[c];
-        sh[(q++) * 64 + lane] = S.sig[c];
-    }
-#pragma unroll
-    for (int c = 0; c < 9; ++c) sh[(q++) * 64 + lane] = S.V[c];
-}
-template <int NM, typename R>
-__device__ __forceinline__ void sst_load(const R* sh, int lane, SSt<NM, R>& S) {
-    int q = 0;
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        S.al[m] = sh[(q++) * 64 + lane];
-        S.ar[m] = sh[(q++) * 64 + lane];
-        S.are[m] = sh[(q++) * 64 + lane];
-    }
-    S.rho = sh[(q++) * 64 + lane];
-    S.E = sh[(q++) * 64 + lane];
-    S.p = sh[(q++) * 64 + lane];
-    S.a = sh[(q++) * 64 + lane];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        S.u[c] = sh[(q++) * 64 + lane];
-        S.sig[c] = sh[(q++) * 64 + lane];
-    }
-#pragma unroll
-    for (int c = 0; c < 9; ++c) S.V[c] = sh[(q++) * 64 + lane];
-}
-
-// y / z pass of the solid path: lanes along x (coalesced), marching along D
-// over a segment of faces.  The right state of row r-1 waits for face r in
-// the wave's own LDS slice (not in registers).  The primitive rows slide:
-// rows r-1 and r stay in registers and row r+1 is the one load per row.
-// Reloading all three rows from cache missed the L2 (a 4 MB L2 per XCD
-// against the rows of all resident waves): 565 B/cell of HBM traffic against
-// 336, which made the FP32 (mixed) pass bandwidth-bound (measured: FP32 pass
-// 1.6 -> 1.1 ms, FP64 3.2 -> 3.0 ms on 256^3).
 template <int NM, int D, bool RW, typename R>
-__device__ __forceinline__ void flux_lmarch_s_body(const Level& lv, const MF& U, const FacesT<R>& F, int seglen, Clock* clk) {
-    if (clk->done) return;
-    constexpr int NF = 3 * NM + 17;
-    constexpr int NS = SStSlots<NM, R>::N;
-    __shared__ R shm[4 * NS * 64];
-    const int lane = threadIdx.x & 63;
-    R* sh = shm + wave_in_block() * NS * 64;
-    const long long wave = (long long)blockIdx.x * (blockDim.x >> 6) + wave_in_block();
-    const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
-    const int nd = lv.n[D];
-    const int no = (D == 1) ? nz : ny;
-    const int nstrip = (nx + 63) / 64;
-    const int nseg = (nd + 1 + seglen - 1) / seglen;
-    if (wave >= (long long)nstrip * nseg * no) return;  // uniform per wave; no block barrier below
-    const int strip = (int)(wave % nstrip);
-    const long long rest = wave / nstrip;
-    const int seg = (int)(rest % nseg);
-    const int o = (int)(rest / nseg);
-    const int i0 = strip * 64 + lane;
-    const bool act = i0 < nx;
-    const int i = act ? i0 : nx - 1;
-    const int f0 = seg * seglen;
-    const int f1 = min(f0 + seglen, nd + 1);
-    const int rb = max(f0 - 1, 0), re = min(f1 - 1, nd - 1);
-    auto cj = [&](int r) { return D == 1 ? r : o; };
-    auto ck = [&](int r) { return D == 2 ? r : o; };
-    auto faceidx = [&](int r) {
-        return D == 1 ? ((long long)ck(r) * (ny + 1) + r) * nx + i : ((long long)r * ny + cj(r)) * nx + i;
-    };
-    unsigned st = 0;
-    // reconstruct row r (MUSCL on rows r-1, r, r+1; p2c and sound speed)
-    auto recon = [&](int r, SSt<NM, R>& SL, SSt<NM, R>& SR) {
-        SPrim<NM, R> Pm, Pc, Pp, PL, PR;
-        load_sprim<NM, R>(lv, U, i, cj(r - 1), ck(r - 1), Pm);
-        load_sprim<NM, R>(lv, U, i, cj(r), ck(r), Pc);
-        load_sprim<NM, R>(lv, U, i, cj(r + 1), ck(r + 1), Pp);
-        muscl_s<NM, R>(Pm, Pc, Pp, PL, PR);
-        p2c_sound_s<NM, RW, R>(lv, PL, D, SL);
-        p2c_sound_s<NM, RW, R>(lv, PR, D, SR);
-    };
-    auto emit = [&](int face, const SSt<NM, R>& A, const SSt<NM, R>& B) {
-        R Fv[NF];
-        wave5<NM, RW, R>(lv, A, B, D, Fv, st);
-        if (!act) return;
-        const long long fi = faceidx(face);
+__global__ __launch_bounds__(256) void k_flux_yz_s(Level lv, MF U, FacesT<R> F, Clock* clk) {
+    using T = STile<NM, R>;
+    constexpr int TC = T::TC, LN = T::LN, PER = T::PER, ROWS = T::ROWS, NF = T::NF, FR = T::FR;
+    __shared__ R lds[T::WORDS];
+    if (clk->done) return;  // uniform: the clock does not change during the launch
+    const int nx = lv.n[0], ny = lv.n[1], nd = lv.n[D];
+    const int nxt = (nx + TC - 1) / TC, nseg = (nd + 1 + PER - 1) / PER;
+    const long long tile = xcd_block(blockIdx.x, gridDim.x, 2);
+    const int xt = (int)(tile % nxt);
+    const int rest = (int)(tile / nxt);
+    const int seg = rest % nseg, o = rest / nseg;
+    const int i0 = xt * TC, c0 = seg * PER - 1;
+    const int tid = threadIdx.x;
+    auto P = [&](int q, int col, int t) -> R& { return lds[(q * TC + col) * ROWS + t]; };
+    // one cell of the first 16 rows per thread; then the two rows left, their
+    // components dealt out over the block, so that all loads are in flight
+    // together (a second round of whole cells leaves 7 threads in 8 idle)
+    {
+        const int col = tid % TC, t = tid / TC, r = c0 - 1 + t;
+        SPrim<NM, R> Pq;
+        load_sprim<NM, R>(lv, U, i0 + col, D == 1 ? r : o, D == 2 ? r : o, Pq);
+        const int hc = tid % TC, ht = LN + (tid / TC & 1), hr = c0 - 1 + ht;
+        int hi = i0 + hc, hj = D == 1 ? hr : o, hk = D == 2 ? hr : o;
+        bool f[3];
+        map3(lv, hi, hj, hk, f);
+        constexpr int HN = (T::NP + 7) / 8;
+        R hv[HN];
 #pragma unroll
-        for (int q = 0; q < NF; ++q) F.p[q * F.cs + fi] = Fv[q];
-    };
-    constexpr bool SLIDE = true;
-    SPrim<NM, R> W0, W1;  // rows r-1 and r (sliding form)
-    if (SLIDE) {
-        load_sprim<NM, R>(lv, U, i, cj(rb - 1), ck(rb - 1), W0);
-        load_sprim<NM, R>(lv, U, i, cj(rb), ck(rb), W1);
-    }
-    for (int r = rb; r <= re; ++r) {
-        SSt<NM, R> SLs, SRs;
-        if (SLIDE) {
-            SPrim<NM, R> W2, PL, PR;
-            load_sprim<NM, R>(lv, U, i, cj(r + 1), ck(r + 1), W2);
-            muscl_s<NM, R>(W0, W1, W2, PL, PR);
-            p2c_sound_s<NM, RW, R>(lv, PL, D, SLs);
-            p2c_sound_s<NM, RW, R>(lv, PR, D, SRs);
-            W0 = W1;
-            W1 = W2;
-        } else {
-            recon(r, SLs, SRs);
-        }
-        if (r >= f0) {  // face r: left UR(r-1) (the image of UR(0) at the domain face), right UL(r)
-            SSt<NM, R> A;
-            if (r == 0) {
-                A = SRs;
-                if (lv.bc_lo[D]) flip_s<NM, R>(A, D);
-            } else {
-                sst_load<NM, R>(sh, lane, A);
+        for (int n = 0; n < HN; ++n) {
+            const int q = tid / 32 + 8 * n;
+            if (q < T::NP) {
+                const bool ep = q >= 2 * NM && q < 3 * NM;
+                const int u = q - 3 * NM;
+                const int comp = q < NM ? lv.cs[ALPHA] + q
+                               : q < 2 * NM ? lv.cs[RHO_K] + q - NM
+                               : ep ? (lv.plastic ? lv.cs[EPSILON] + q - 2 * NM : 0)
+                               : u < 3 ? lv.cs[VELOCITY] + u
+                               : u == 3 ? lv.cs[PRESSURE] : lv.cs[V_TENSOR] + u - 4;
+                const R v = (R)U.at(comp, hi, hj, hk);
+                hv[n] = ep && !lv.plastic ? R(0) : ((u == 0 && f[0]) || (u == 1 && f[1]) || (u == 2 && f[2]) ? -v : v);
             }
-            emit(r, A, SLs);
         }
-        sst_store<NM, R>(sh, lane, SRs);
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            P(m, col, t) = Pq.a[m];
+            P(NM + m, col, t) = Pq.r[m];
+            P(2 * NM + m, col, t) = Pq.e[m];
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) P(3 * NM + q, col, t) = Pq.u[q];
+        P(3 * NM + 3, col, t) = Pq.p;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) P(3 * NM + 4 + q, col, t) = Pq.V[q];
+#pragma unroll
+        for (int n = 0; n < HN; ++n) {
+            const int q = tid / 32 + 8 * n;
+            if (q < T::NP) P(q, hc, ht) = hv[n];
+        }
     }
-    if (f1 == nd + 1) {  // domain face nd: UR(nd-1) and the image of UL(nd-1)
-        SSt<NM, R> SLs, SRs;
-        recon(nd - 1, SLs, SRs);
-        if (lv.bc_hi[D]) flip_s<NM, R>(SLs, D);
-        emit(nd, SRs, SLs);
+    __syncthreads();
+    const int ld = tid % LN, col = tid / LN;
+    const int c = c0 + ld;  // the lane's cell along D
+    bool fl;
+    const int s = bcmap(c, nd, lv.bc_lo[D], lv.bc_hi[D], fl);
+    SPrim<NM, R> PL, PR;
+    {
+        // row s of the tile (lanes beyond the domain hold no face: clamped)
+        const int t = min(max(s - c0 + 1, 1), ROWS - 2);
+        auto get = [&](int tt, SPrim<NM, R>& Pq) {
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                Pq.a[m] = P(m, col, tt);
+                Pq.r[m] = P(NM + m, col, tt);
+                Pq.e[m] = P(2 * NM + m, col, tt);
+            }
+#pragma unroll
+            for (int q = 0; q < 3; ++q) Pq.u[q] = P(3 * NM + q, col, tt);
+            Pq.p = P(3 * NM + 3, col, tt);
+#pragma unroll
+            for (int q = 0; q < 9; ++q) Pq.V[q] = P(3 * NM + 4 + q, col, tt);
+        };
+        SPrim<NM, R> Pm, Pc, Pp;
+        get(t - 1, Pm);
+        get(t, Pc);
+        get(t + 1, Pp);
+        muscl_s<NM, R>(Pm, Pc, Pp, PL, PR);
+    }
+    unsigned st = 0;
+    R Fv[NF];
+    const bool face = i0 + col < nx && ld >= 1 && c >= 0 && c <= nd;
+    face_s<NM, D, RW, R>(lv, PL, PR, c, face, Fv, st);
+    __syncthreads();  // every wave has read its primitives: the fluxes may overwrite them
+    if (face) {
+#pragma unroll
+        for (int q = 0; q < NF; ++q) lds[(q * TC + col) * FR + ld - 1] = Fv[q];
+    }
+    __syncthreads();
+    {
+        const int cc = tid % TC, f = tid / TC;  // column, face of the segment
+        const int ii = i0 + cc, cf = c0 + 1 + f;
+        if (f < PER && ii < nx && cf <= nd) {
+            const int fj = D == 1 ? cf : o, fk = D == 2 ? cf : o;
+            const long long id = ((long long)fk * F.ny + fj) * F.nx + ii;
+#pragma unroll
+            for (int q = 0; q < NF; ++q) F.p[q * F.cs + id] = lds[(q * TC + cc) * FR + f];
+        }
     }
     if (st) atomicOr(&clk->status, st);
-}
-template <int NM, int D, bool RW, typename R>
-__global__ __launch_bounds__(256) void k_flux_lmarch_s(Level lv, MF U, FacesT<R> F, int seglen, Clock* clk) {
-    flux_lmarch_s_body<NM, D, RW, R>(lv, U, F, seglen, clk);
 }
 
 // Per-cell solid state held by the update kernel.

@@ -4,7 +4,7 @@
 // to per-material EOS / plasticity parameters (Gamma0, s, yield stress; for
 // fluids the Gruneisen coefficient adiabaticIndex - 1 and pref).  Each kernel mirrors
 // its FP64 counterpart (k_init_p2c_s, k_sound_dt_s, k_flux_x_s /
-// k_flux_lmarch_s, k_update_s, k_clock_dt, k_clock_advance) operation for
+// k_flux_yz_s, k_update_s, k_clock_dt, k_clock_advance) operation for
 // operation, so the value parts equal the FP64 trajectory bit for bit.
 //
 // Layout: a state's values are the caller's CellArray; its derivative parts

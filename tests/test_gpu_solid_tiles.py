@@ -1,0 +1,48 @@
+"""Solid flux passes at the edges of their tiles: segments of 64 or 32 lanes
+along x, tiles of 16 columns by 15 faces along y and z, ragged rows, and
+reflective ends.  The FP64 state must equal the oracle's bit for bit."""
+from __future__ import annotations
+
+import dataclasses
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _plate(n, bc_lo=(0, 0, 0), bc_hi=(0, 0, 0), box=16):
+    """The plate impact cut down to n cells of the same size."""
+    from tenjin_amd import configs
+
+    dim = len(n)
+    m = max(n)
+    pb = configs.plate_impact(dim=dim, n=m, box=box, length=25.6e-3 * m / 256)
+    nx, ny, nz = (tuple(n) + (1,))[:3]
+    lo = [(m - q) // 2 for q in (nx, ny)] + [0]
+    prims = pb.prims[:, lo[2]:lo[2] + nz, lo[1]:lo[1] + ny, lo[0]:lo[0] + nx]
+    return dataclasses.replace(pb, n=(nx, ny, nz), L=tuple(1e-4 * q for q in (nx, ny, nz)), bc_lo=bc_lo, bc_hi=bc_hi,
+                               prims=np.ascontiguousarray(prims))
+
+
+@pytest.mark.parametrize("n,bc", [
+    ((14, 15), 0), ((15, 14), 1), ((16, 16), 0), ((17, 29), 1), ((30, 30), 0), ((31, 31), 1), ((62, 13), 0),
+    ((63, 32), 1), ((64, 44), 0), ((95, 3), 0), ((3, 46), 1), ((16, 14, 15), 0), ((33, 17, 14), 1), ((5, 31, 16), 0)])
+def test_solid_tiles_match_oracle(n, bc):
+    from oracle.oracle import Oracle
+    from tenjin_amd import GpuLevel
+
+    pb = _plate(n, bc_lo=(bc, 0, bc), bc_hi=(0, bc, bc))
+    print(f"\n[case] solid tiles {n} bc {bc}", flush=True)
+    o, g = Oracle(pb), GpuLevel(pb)
+    g.init_from_prims(pb.prims, pb.shift_pressure)
+    for step in range(4):
+        dt = o.driver_dt(step, 0.0)
+        assert g.compute_dt() * (0.2 if step < 5 else 1.0) == dt
+        o.step(dt)
+        g.set_dt(dt, reset_clock=1)
+        g.step()
+        ref, got = o.get(), g.get_state()
+        for c in pb.layout.state_comps():
+            assert np.array_equal(ref[c], got[c]), (step, pb.layout.names[c])
+    assert g.status() == 0
