@@ -45,7 +45,7 @@ struct tj_ctx {
     int ncu = 0;  // compute units of the device
     std::map<std::pair<const void*, int>, int> seg_cache;
     bool fuse = false;
-    // two-dimensional fluid levels without a mixture: each RK stage as the x
+    // two-dimensional fluid levels: each RK stage as the x
     // and y stage kernels (tj_stage2d.h) over the partially updated state
     // d_ux, with no flux planes (on by default; off: the flux-plane passes)
     bool stage2d = true;

@@ -411,8 +411,10 @@ static int make_level(std::string& err, const tj_level_desc* d, Level& lv, std::
     return TJ_OK;
 }
 
-// A level the stage kernels serve: two-dimensional fluid, no mixture.
-static bool stage2d_level(const tj_ctx* c) { return !c->lv.solid && c->lv.dim == 2 && c->lv.mixm < 0; }
+// A level the stage kernels serve: two-dimensional fluid.
+static bool stage2d_level(const tj_ctx* c) { return !c->lv.solid && c->lv.dim == 2; }
+// components of the partially updated state between their two kernels
+static int ux_comps(const tj_ctx* c) { return 2 * c->nmat + 4 + (c->lv.mixm >= 0 ? 1 : 0); }
 
 int tj_bind_level(tj_ctx* c, const tj_level_desc* d) {
     if (!c || !d) return TJ_EINVAL;
@@ -446,7 +448,14 @@ int tj_bind_level(tj_ctx* c, const tj_level_desc* d) {
         F.p = c->d_flux[a];
         c->estride[a] = F.cs;
     }
-    if (stage2d_level(c)) HIPCHK(c, hipMalloc(&c->d_ux, sizeof(double) * lv.ncells * (2 * d->nmat + 4)));
+    if (stage2d_level(c)) {
+        const hipError_t e = hipMalloc(&c->d_ux, sizeof(double) * lv.ncells * ux_comps(c));
+        if (e != hipSuccess) {  // a mixture's stages also run on the flux planes
+            c->d_ux = nullptr;
+            (void)hipGetLastError();
+            if (lv.mixm < 0) HIPCHK(c, e);
+        }
+    }
     if (d->THINC) {
         const long long pl = lv.ncells * d->nmat;
         HIPCHK(c, hipMalloc(&c->d_urstar, sizeof(double) * pl));
@@ -882,7 +891,7 @@ extern "C++" {
 #ifndef TJ_STAGE_LPS
 #define TJ_STAGE_LPS 16
 #endif
-template <bool TH, typename R>
+template <bool TH, typename R, bool MX>
 static void launch_stage2d_t(tj_ctx* c, int stage, const MF& in, const MF& base, const MF& out, unsigned ops,
                              const Hist& hx, const Hist& hy, const char* nx_name, const char* ny_name) {
     constexpr int TC = TJ_STAGE_TC;
@@ -892,7 +901,7 @@ static void launch_stage2d_t(tj_ctx* c, int stage, const MF& in, const MF& base,
         Timed tm(c, nx_name);
         constexpr int CPW = XGeom<TH>::CPW;
         const long long waves = (long long)((lv.n[0] + CPW - 1) / CPW) * lv.n[1];
-        hipLaunchKernelGGL((k_xstage<2, TH, R>), dim3(grid1(waves, 4)), dim3(256), 0, c->stream, lv, in, ux, hx, c->d_clk);
+        hipLaunchKernelGGL((k_xstage<2, TH, R, MX>), dim3(grid1(waves, 4)), dim3(256), 0, c->stream, lv, in, ux, hx, c->d_clk);
     }
     if (TH) {
         c->pass += 1;
@@ -904,10 +913,10 @@ static void launch_stage2d_t(tj_ctx* c, int stage, const MF& in, const MF& base,
         constexpr int CPW = YTile<2, TH, TC, LPS, R>::CPW;
         const long long tiles = (long long)((lv.n[0] + TC - 1) / TC) * ((lv.n[1] + CPW - 1) / CPW);
         if (stage == 1)
-            hipLaunchKernelGGL((k_ystage<2, TH, TC, LPS, 1, R>), dim3((unsigned)tiles), dim3(TC * LPS), 0, c->stream, lv,
+            hipLaunchKernelGGL((k_ystage<2, TH, TC, LPS, 1, R, MX>), dim3((unsigned)tiles), dim3(TC * LPS), 0, c->stream, lv,
                                in, ux, base, out, hy, c->d_clk, ops);
         else
-            hipLaunchKernelGGL((k_ystage<2, TH, TC, LPS, 2, R>), dim3((unsigned)tiles), dim3(TC * LPS), 0, c->stream, lv,
+            hipLaunchKernelGGL((k_ystage<2, TH, TC, LPS, 2, R, MX>), dim3((unsigned)tiles), dim3(TC * LPS), 0, c->stream, lv,
                                in, ux, base, out, hy, c->d_clk, ops);
     }
     if (TH) {
@@ -930,13 +939,19 @@ static int launch_stage2d(tj_ctx* c, int stage, const MF& in, const MF& base, co
     c->dpass[1] = d1;
     const char* a = xn[mixed][stage - 1];
     const char* b = yn[mixed][stage - 1];
+#define TJ_STAGE2D(TH, R)                                                                            \
+    do {                                                                                            \
+        if (c->lv.mixm >= 0) launch_stage2d_t<TH, R, true>(c, stage, in, base, out, ops, hx, hy, a, b); \
+        else launch_stage2d_t<TH, R, false>(c, stage, in, base, out, ops, hx, hy, a, b);            \
+    } while (0)
     if (c->desc.THINC) {
-        if (mixed) launch_stage2d_t<true, float>(c, stage, in, base, out, ops, hx, hy, a, b);
-        else launch_stage2d_t<true, double>(c, stage, in, base, out, ops, hx, hy, a, b);
+        if (mixed) TJ_STAGE2D(true, float);
+        else TJ_STAGE2D(true, double);
     } else {
-        if (mixed) launch_stage2d_t<false, float>(c, stage, in, base, out, ops, hx, hy, a, b);
-        else launch_stage2d_t<false, double>(c, stage, in, base, out, ops, hx, hy, a, b);
+        if (mixed) TJ_STAGE2D(false, float);
+        else TJ_STAGE2D(false, double);
     }
+#undef TJ_STAGE2D
     HIPCHK(c, hipGetLastError());
     return TJ_OK;
 }
@@ -1629,8 +1644,9 @@ struct Carve {
 };
 
 // The buffers of tj_bind_level for a level, carved from `base` (or only
-// measured, base == null): returns the bytes used.
-size_t carve_level(tj_ctx* c, const tj_level_desc* d, unsigned char* base, int prec) {
+// measured, base == null): returns the bytes used.  ux: with the stage
+// kernels' planes (a mixture's stages run on the flux planes without them).
+size_t carve_level(tj_ctx* c, const tj_level_desc* d, unsigned char* base, int prec, bool ux) {
     Carve cv{base};
     Level& lv = c->lv;
     c->d_clk = cv.take<Clock>(1);
@@ -1661,7 +1677,7 @@ size_t carve_level(tj_ctx* c, const tj_level_desc* d, unsigned char* base, int p
             G.p = c->d_fluxf[a];
         }
     }
-    if (stage2d_level(c)) c->d_ux = cv.take<double>(lv.ncells * (2 * d->nmat + 4));
+    c->d_ux = ux && stage2d_level(c) ? cv.take<double>(lv.ncells * ux_comps(c)) : nullptr;
     if (d->THINC) {
         const long long pl = lv.ncells * d->nmat;
         c->d_urstar = cv.take<double>(pl);
@@ -1705,7 +1721,11 @@ extern "C" int tj_run_static(const tj_level_desc* desc, tj_mf* S, tj_mf* T, doub
     if (r) return r;
     c->desc = *desc;
     c->nmat = desc->nmat;
-    if (carve_level(c, desc, nullptr, prec) > (size_t)TJ_STATIC_SCRATCH_BYTES) return TJ_ESCRATCH;
+    bool ux = true;
+    if (carve_level(c, desc, nullptr, prec, ux) > (size_t)TJ_STATIC_SCRATCH_BYTES) {
+        ux = false;
+        if (c->lv.mixm < 0 || carve_level(c, desc, nullptr, prec, ux) > (size_t)TJ_STATIC_SCRATCH_BYTES) return TJ_ESCRATCH;
+    }
     int ncomp_cs[NVAR];
     const int ncomp = build_layout(*desc, ncomp_cs);
     const Level& lv = c->lv;
@@ -1718,7 +1738,7 @@ extern "C" int tj_run_static(const tj_level_desc* desc, tj_mf* S, tj_mf* T, doub
     if (hipGetDevice(&dev) != hipSuccess) return TJ_EHIP;
     unsigned char* base = nullptr;
     if ((r = scratch_for_device(dev, &base))) return r;
-    carve_level(c, desc, base, prec);
+    carve_level(c, desc, base, prec, ux);
     c->device = dev;
     c->stream = static_cast<hipStream_t>(stream);
     c->seglen = 16;  // fixed segment length: the per-pass pick keeps a host-side cache

@@ -32,7 +32,8 @@ inline namespace TJ_VIEW_NS {
 
 // Partially updated conserved state between the two kernels of a stage:
 // component-major planes of FP64 over the level's cells, in the order
-// alpha (NM), alpha rho (NM), rho u (3), E.
+// alpha (NM), alpha rho (NM), rho u (3), E and, with a mixture, alpha rho
+// lambda.
 struct UxPlanes {
     double* p;
     long long cs;  // component stride (= cells)
@@ -56,10 +57,10 @@ struct XFin {
     MF Ub, Uo;
     unsigned ops;
 };
-template <int NM, bool TH, typename R, int FIN = 0>
+template <int NM, bool TH, typename R, int FIN = 0, bool MX = false>
 __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const UxPlanes& Ux, const Hist& h, Clock* clk,
                                             long long wave, const XFin& fin = XFin{}) {
-    constexpr int NF = 2 * NM + 5;
+    constexpr int NF = 2 * NM + 5 + (MX ? 1 : 0);  // flux components per face
     if (clk->done) return;
     constexpr int H = XGeom<TH>::H, CPW = XGeom<TH>::CPW;
     const int lane = threadIdx.x & 63;
@@ -75,10 +76,10 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
     const int lofs = s - c;
 
     Prim<NM, R> Pm, Pc, Pp, PL, PR;
-    load_prim<NM, R>(lv, U, s - 1, j, k, Pm);
-    load_prim<NM, R>(lv, U, s, j, k, Pc);
-    load_prim<NM, R>(lv, U, s + 1, j, k, Pp);
-    muscl<NM, R>(Pm, Pc, Pp, PL, PR);
+    load_prim<NM, R, MX>(lv, U, s - 1, j, k, Pm);
+    load_prim<NM, R, MX>(lv, U, s, j, k, Pc);
+    load_prim<NM, R, MX>(lv, U, s + 1, j, k, Pp);
+    muscl<NM, R, MX>(Pm, Pc, Pp, PL, PR);
 
     unsigned st = 0;
     const long long cell_s = (long long)j * nx + s;
@@ -137,8 +138,8 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
     }
 
     FSt<NM, R> SLs, SRs;
-    p2c_sound<NM, R>(lv, PL, SLs);
-    p2c_sound<NM, R>(lv, PR, SRs);
+    p2c_sound<NM, R, MX>(lv, PL, SLs);
+    p2c_sound<NM, R, MX>(lv, PR, SRs);
 
     // left state of face c: UR(c-1) from the neighbouring lane
     FSt<NM, R> Lf;
@@ -153,6 +154,7 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
     Lf.E = lane_dn(SRs.E);
     Lf.p = lane_dn(SRs.p);
     Lf.a = lane_dn(SRs.a);
+    if (MX) Lf.arl = lane_dn(SRs.arl);
 
     // face c: lanes H .. H + CPW (faces s0 .. s0 + CPW), up to the domain's top face
     const bool face = lane >= H && lane <= H + CPW && c >= 0 && c <= nx;
@@ -167,7 +169,7 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
         FSt<NM, R> Rf = SLs;
         if (c == nx && lv.bc_hi[0]) flip_state<NM, R>(Rf, 0);
         R sa[NM];
-        hllc<NM, R>(Lf, Rf, 0, Fv, sa);
+        hllc<NM, R, MX>(Lf, Rf, 0, Fv, sa);
         if (TH && (c < s0 + CPW || c == nx)) {
             if (c < nx) {
 #pragma unroll
@@ -186,11 +188,11 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
     double cand = __builtin_huge_val();
     if (own) {
         const long long cell = (long long)j * nx + c;
-        double al[NM], ar[NM], ru[3], E, a0[NM];
-        load_cons<NM>(lv, U, c, j, k, al, ar, ru, E);
+        double al[NM], ar[NM], ru[3], E, a0[NM], arl = 0.0;
+        load_cons<NM, MX>(lv, U, c, j, k, al, ar, ru, E, &arl);
 #pragma unroll
         for (int m = 0; m < NM; ++m) a0[m] = al[m];
-        accum_dir<NM, R>(al, ar, ru, E, a0, clk->dt / lv.dx[0], Fv, Fh);
+        accum_dir<NM, R, MX>(al, ar, ru, E, a0, clk->dt / lv.dx[0], Fv, Fh, &arl);
         if constexpr (FIN == 0) {
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
@@ -200,8 +202,9 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
 #pragma unroll
             for (int q = 0; q < 3; ++q) Ux.at(2 * NM + q, cell) = ru[q];
             Ux.at(2 * NM + 3, cell) = E;
+            if (MX) Ux.at(2 * NM + 4, cell) = arl;
         } else {
-            finish_cell<NM, FIN>(lv, fin.Ub, fin.Uo, c, j, k, al, ar, ru, E, clk->dt, fin.ops, cand, st);
+            finish_cell<NM, FIN, MX>(lv, fin.Ub, fin.Uo, c, j, k, al, ar, ru, E, clk->dt, fin.ops, cand, st, arl);
         }
     }
     if constexpr (FIN == 2) {
@@ -210,12 +213,12 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
     if (st) atomicOr(&clk->status, st);
 }
 
-template <int NM, bool TH, typename R = double>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && sizeof(R) == 8 ? 4 : 1)))
+template <int NM, bool TH, typename R = double, bool MX = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && !MX && sizeof(R) == 8 ? 4 : 1)))
 void k_xstage(Level lv, MF U, UxPlanes Ux, Hist h, Clock* clk) {
     const long long nb = gridDim.x;
     const long long b = xcd_block(blockIdx.x, nb, 2);
-    xstage_body<NM, TH, R>(lv, U, Ux, h, clk, b * (blockDim.x >> 6) + wave_in_block());
+    xstage_body<NM, TH, R, 0, MX>(lv, U, Ux, h, clk, b * (blockDim.x >> 6) + wave_in_block());
 }
 
 // One RK stage of a one-dimensional fluid level in one launch (FIN = STAGE).
@@ -257,13 +260,13 @@ void k_xstage1d(Level lv, MF U, MF Ub, MF Uo, Hist h, Clock* clk, unsigned ops, 
 // loads after its barrier overlap the others' arithmetic: lane l of a
 // segment holds row r = s0 - H + l, the segment computes faces s0 .. s0 + CPW
 // and completes cells s0 .. s0 + CPW - 1.
-template <int NM, bool TH, int TC, int LPS, typename R>
+template <int NM, bool TH, int TC, int LPS, typename R, bool MX = false>
 struct YTile {
     static constexpr int H = TH ? 2 : 1;
     static constexpr int CPW = LPS - 2 * H;    // rows completed per tile
-    static constexpr int NP = 2 * NM + 4;      // staged primitives: alpha, rho_k, u (3), p
+    static constexpr int NP = 2 * NM + 4 + (MX ? 1 : 0);  // staged primitives: alpha, rho_k, u (3), p, lambda
     static constexpr int ROWS = LPS + 2;       // rows s0 - H - 1 .. s0 - H + LPS
-    static constexpr int NF = 2 * NM + 5;      // flux components per face
+    static constexpr int NF = 2 * NM + 5 + (MX ? 1 : 0);  // flux components per face
     static constexpr int FR = CPW + 1;         // faces per column
     static constexpr int NT = TC * LPS;        // threads per block
     static constexpr int NW = NT / 64;         // waves per block
@@ -287,10 +290,10 @@ __device__ __forceinline__ void block_min_to_n(double cand, unsigned long long* 
     }
 }
 
-template <int NM, bool TH, int TC, int LPS, int STAGE, typename R>
+template <int NM, bool TH, int TC, int LPS, int STAGE, typename R, bool MX = false>
 __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const UxPlanes& Ux, const MF& Ub,
                                             const MF& Uo, const Hist& h, Clock* clk, unsigned ops, long long tile) {
-    using T = YTile<NM, TH, TC, LPS, R>;
+    using T = YTile<NM, TH, TC, LPS, R, MX>;
     constexpr int H = T::H, CPW = T::CPW, NP = T::NP, ROWS = T::ROWS, NF = T::NF, FR = T::FR, NT = T::NT;
     __shared__ R lds[T::WORDS];
     __shared__ unsigned long long red[T::NW];
@@ -309,10 +312,39 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
     auto FL = [&](int q, int col, int f) -> R& { return lds[(q * TC + col) * FR + f]; };
 
     // ---- stage the tile's primitives (load_prim of every LDS row and column)
-    for (int e = tid; e < ROWS * TC; e += NT) {
-        const int col = e % TC, t = e / TC;
+    // one cell of the first LPS rows per thread, then the two rows left with
+    // their components (and with THINC the neighbouring columns' alphas) dealt
+    // out over the block, so that all loads are in flight together (whole cells
+    // in a second and third round: FP64 2048 x 1024 179 / 225 us a stage, 174 /
+    // 218 now; mixed 138 / 187 and 135 / 182)
+    {
+        const int col = tid % TC, t = tid / TC;
         Prim<NM, R> Pq;
-        load_prim<NM, R>(lv, U, i0 + col, base + t, 0, Pq);
+        load_prim<NM, R, MX>(lv, U, i0 + col, base + t, 0, Pq);
+        // items of the second part: NP * 2 * TC halo values, then NM * 2 * ROWS alphas
+        constexpr int HV = NP * 2 * TC, AV = TH ? NM * 2 * ROWS : 0, HN = (HV + AV + NT - 1) / NT;
+        R hv[HN];
+#pragma unroll
+        for (int n = 0; n < HN; ++n) {
+            const int e = tid + n * NT;
+            if (e < HV + AV) {
+                const bool al = e >= HV;
+                const int a = e - HV;
+                const int q = al ? a / (2 * ROWS) : e / (2 * TC);  // component, or material of an alpha
+                const int w = al ? a % (2 * ROWS) : e % (2 * TC);
+                int ii = al ? ((w & 1) ? i0 + TC : i0 - 1) : i0 + w % TC;
+                int jj = base + (al ? w >> 1 : LPS + w / TC), kk = 0;
+                bool f[3];
+                map3(lv, ii, jj, kk, f);
+                const int u = q - 2 * NM;
+                const int comp = (al || q < NM) ? lv.cs[ALPHA] + q
+                               : q < 2 * NM ? lv.cs[RHO_K] + q - NM
+                               : u < 3 ? lv.cs[VELOCITY] + u
+                               : !MX || u == 3 ? lv.cs[PRESSURE] : lv.cs[LAMBDA];
+                const R v = (R)U.at(comp, ii, jj, kk);
+                hv[n] = !al && ((u == 0 && f[0]) || (u == 1 && f[1])) ? -v : v;
+            }
+        }
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             P(m, col, t) = Pq.a[m];
@@ -321,12 +353,12 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
 #pragma unroll
         for (int q = 0; q < 3; ++q) P(2 * NM + q, col, t) = Pq.u[q];
         P(2 * NM + 3, col, t) = Pq.p;
-    }
-    if (TH) {
-        for (int e = tid; e < ROWS * 2; e += NT) {
-            const int side = e & 1, t = e >> 1;
+        if (MX) P(2 * NM + 4, col, t) = Pq.lam;
 #pragma unroll
-            for (int m = 0; m < NM; ++m) AX(m, side, t) = load_alpha<R>(lv, U, m, side ? i0 + TC : i0 - 1, base + t, 0);
+        for (int n = 0; n < HN; ++n) {
+            const int e = tid + n * NT;
+            if (e < HV) P(e / (2 * TC), e % TC, LPS + e % (2 * TC) / TC) = hv[n];
+            else if (e < HV + AV) AX((e - HV) / (2 * ROWS), (e - HV) & 1, (e - HV) % (2 * ROWS) >> 1) = hv[n];
         }
     }
     __syncthreads();
@@ -356,6 +388,7 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
 #pragma unroll
         for (int q = 0; q < 3; ++q) Pq.u[q] = P(2 * NM + q, col, t);
         Pq.p = P(2 * NM + 3, col, t);
+        if (MX) Pq.lam = P(2 * NM + 4, col, t);
     };
     // load_alpha of (i + di, g): the tile's own column or a neighbouring one
     auto alpha_at = [&](int m, int di, int g) -> R {
@@ -371,7 +404,7 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
     prim_at(s - 1, Pm);
     prim_at(s, Pc);
     prim_at(s + 1, Pp);
-    muscl<NM, R>(Pm, Pc, Pp, PL, PR);
+    muscl<NM, R, MX>(Pm, Pc, Pp, PL, PR);
 
     unsigned st = 0;
     const long long cell_s = (long long)s * nx + i;
@@ -461,8 +494,8 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
     }
 
     FSt<NM, R> SLs, SRs;
-    p2c_sound<NM, R>(lv, PL, SLs);
-    p2c_sound<NM, R>(lv, PR, SRs);
+    p2c_sound<NM, R, MX>(lv, PL, SLs);
+    p2c_sound<NM, R, MX>(lv, PR, SRs);
     // UR of the row below from lane - 1; the segment's first lane takes the
     // previous segment's value, but it is a halo lane (sl = 0 < H) whose Lf is
     // never read
@@ -478,6 +511,7 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
     Lf.E = lane_dn(SRs.E);
     Lf.p = lane_dn(SRs.p);
     Lf.a = lane_dn(SRs.a);
+    if (MX) Lf.arl = lane_dn(SRs.arl);
 
     const bool face = colok && sl >= H && sl <= H + CPW && r >= 0 && r <= ny;
     R Fv[NF];
@@ -491,7 +525,7 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
         FSt<NM, R> Rf = SLs;
         if (r == ny && lv.bc_hi[1]) flip_state<NM, R>(Rf, 1);
         R sa[NM];
-        hllc<NM, R>(Lf, Rf, 1, Fv, sa);
+        hllc<NM, R, MX>(Lf, Rf, 1, Fv, sa);
         if (TH && (r < s0 + CPW || r == ny)) {
             if (r < ny) {
 #pragma unroll
@@ -518,7 +552,7 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
         const int ii = i0 + cc, rr = s0 + f;
         if (ii < nx && rr < ny) {
             const long long cell = (long long)rr * nx + ii;
-            double al[NM], ar[NM], ru[3], E, a0[NM];
+            double al[NM], ar[NM], ru[3], E, a0[NM], arl = 0.0;
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
                 al[m] = Ux.at(m, cell);
@@ -528,14 +562,15 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
 #pragma unroll
             for (int q = 0; q < 3; ++q) ru[q] = Ux.at(2 * NM + q, cell);
             E = Ux.at(2 * NM + 3, cell);
+            if (MX) arl = Ux.at(2 * NM + 4, cell);
             R Flo[NF], Fhi[NF];
 #pragma unroll
             for (int q = 0; q < NF; ++q) {
                 Flo[q] = FL(q, cc, f);
                 Fhi[q] = FL(q, cc, f + 1);
             }
-            accum_dir<NM, R>(al, ar, ru, E, a0, dt / lv.dx[1], Flo, Fhi);
-            finish_cell<NM, STAGE>(lv, Ub, Uo, ii, rr, 0, al, ar, ru, E, dt, ops, cand, st);
+            accum_dir<NM, R, MX>(al, ar, ru, E, a0, dt / lv.dx[1], Flo, Fhi, &arl);
+            finish_cell<NM, STAGE, MX>(lv, Ub, Uo, ii, rr, 0, al, ar, ru, E, dt, ops, cand, st, arl);
         }
     }
     if (STAGE == 2 && (ops & 8u)) block_min_to_n<T::NW>(cand, dt_slot(lv, clk), red);
@@ -545,13 +580,16 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
 // The mixed form's y kernels take six waves per SIMD (71 VGPRs in stage 2,
 // from 95, no spill): stage 2 0.211 -> 0.202 ms on the 2048 x 1024 level.
 // The FP64 form at five spills about 100 bytes per lane and runs 1.6x slower.
-template <int NM, bool TH, int TC, int LPS, int STAGE, typename R = double>
-__global__ __launch_bounds__(TC * LPS) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 6 : 1))) void k_ystage(Level lv, MF U, UxPlanes Ux, MF Ub, MF Uo, Hist h, Clock* clk,
-                                                     unsigned ops) {
+// With a mixture (MX) the stages cost 1.8 times less than on the flux planes
+// (512 x 256: 209 against 382 us a step), whose y march has one wave per 64
+// columns and 16 rows: 264 waves there.
+template <int NM, bool TH, int TC, int LPS, int STAGE, typename R = double, bool MX = false>
+__global__ __launch_bounds__(TC * LPS) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && !MX ? 6 : 1)))
+void k_ystage(Level lv, MF U, UxPlanes Ux, MF Ub, MF Uo, Hist h, Clock* clk, unsigned ops) {
     // tiles renumbered per XCD (xcd_block): neighbouring column tiles, which
     // share cache lines of rows whose pitch is not a multiple of the line,
     // and the row bands above and below, which share halo rows, run in one L2
-    ystage_body<NM, TH, TC, LPS, STAGE, R>(lv, U, Ux, Ub, Uo, h, clk, ops, xcd_block(blockIdx.x, gridDim.x, 2));
+    ystage_body<NM, TH, TC, LPS, STAGE, R, MX>(lv, U, Ux, Ub, Uo, h, clk, ops, xcd_block(blockIdx.x, gridDim.x, 2));
 }
 
 }  // inline namespace TJ_VIEW_NS

@@ -1,0 +1,73 @@
+"""Two-dimensional levels with a mixture material on the stage kernels: at the
+edges of their tiles (60 / 62 cells along x, 12 / 14 rows along y) against the
+oracle, bit for bit; against the flux-plane passes; and tj_run_static of a
+level whose scratch holds the flux planes but not the stage planes."""
+from __future__ import annotations
+
+import ctypes
+import dataclasses
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _tube(nx, ny, thinc, box=16):
+    from tenjin_amd import configs
+
+    pb = configs.reactive_tube(dim=2, n=max(nx, 2 * ny), box=box, thinc=thinc)
+    prims = np.ascontiguousarray(pb.prims[:, :, :ny, :nx])
+    return dataclasses.replace(pb, n=(nx, ny, 1), prims=prims)
+
+
+@pytest.mark.parametrize("nx,ny,thinc", [(12, 11, 1), (59, 12, 1), (60, 13, 1), (61, 25, 1), (62, 14, 0), (63, 15, 0),
+                                         (17, 29, 0), (33, 24, 1)])
+def test_mixture_stage_tiles_match_oracle(nx, ny, thinc):
+    from oracle.oracle import Oracle
+    from tenjin_amd import GpuLevel
+
+    pb = _tube(nx, ny, thinc)
+    print(f"\n[case] mixture stage tiles {nx} x {ny} thinc {thinc}", flush=True)
+    o, g, f = Oracle(pb), GpuLevel(pb), GpuLevel(pb)
+    f.set_tuning(fuse=0)
+    for q in (g, f):
+        q.init_from_prims(pb.prims)
+    for step in range(4):
+        dt = o.driver_dt(step, 0.0)
+        o.step(dt)
+        for q in (g, f):
+            q.set_dt(dt, reset_clock=1)
+            q.step()
+        ref = o.get()
+        for q in (g, f):
+            got = q.get_state()
+            for c in pb.layout.state_comps():
+                assert np.array_equal(ref[c], got[c]), (step, pb.layout.names[c])
+    assert g.status() == f.status() == o.status()
+
+
+def test_static_scratch_without_stage_planes():
+    import torch
+
+    from tenjin_amd import GpuLevel, LevelDesc, MFView, level_desc, load_library
+
+    pb = _tube(832, 416, 0, box=64)  # flux planes 53 MiB, stage planes 24 MiB more, of 64 MiB
+    print("\n[case] static run, flux planes only", flush=True)
+    L = load_library()
+    mfp = ctypes.POINTER(MFView)
+    L.tj_run_static.argtypes = [ctypes.POINTER(LevelDesc), mfp, mfp, ctypes.c_double, ctypes.c_int, ctypes.c_int,
+                                ctypes.c_int, ctypes.c_void_p, ctypes.POINTER(ctypes.c_double),
+                                ctypes.POINTER(ctypes.c_int)]
+    g = GpuLevel(pb)
+    g.init_from_prims(pb.prims)
+    S, T = g.S.clone(), torch.zeros_like(g.S)
+    torch.cuda.synchronize()
+    n, t = g.run(float("inf"), max_steps=2)
+    vS, vT, d = g._view(S), g._view(T), level_desc(pb)
+    tt, nn = ctypes.c_double(), ctypes.c_int()
+    assert L.tj_run_static(ctypes.byref(d), ctypes.byref(vS), ctypes.byref(vT), float("inf"), 2, 0, 8, None,
+                           ctypes.byref(tt), ctypes.byref(nn)) == 0
+    torch.cuda.synchronize()
+    assert (nn.value, tt.value) == (n, t)
+    assert torch.equal(S, g.S)
