@@ -172,6 +172,34 @@ __device__ __forceinline__ float tdiv(float a, float b) { return a * __builtin_a
 // domain end it is a boundary flux that moves mass and energy in or out.
 __device__ __forceinline__ double tdiv_cr(double a, double b) { return a / b; }
 __device__ __forceinline__ float tdiv_cr(float a, float b) { return a / b; }
+// 1/b by v_rcp_f64 and two Newton steps (a few ulp at worst): the reciprocal
+// that qdiv's quotients and the derivative parts of dual numbers share.
+__device__ __forceinline__ double drcp(double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    double e = __builtin_fma(-b, r, 1.0);
+    r = __builtin_fma(r, e, r);
+    e = __builtin_fma(-b, r, 1.0);
+    return __builtin_fma(r, e, r);
+}
+// a / b correctly rounded, as a / b: the quotient by the reciprocal, corrected
+// by its exact residual (Markstein, IBM J. Res. Dev. 34, 1990), and IEEE's
+// special cases by v_div_fixup_f64.  Written out, so that quotients with one
+// divisor share its reciprocal: 54 cycles a wave for the first and 19 for each
+// further one, against 62 for every a / b, whose sequence also scales both
+// operands by a power of two.  Without the scaling the residual is exact for
+// a = 0 or |a| >= 2^-969 and a divisor in [2^-1021, 2^1021] (and 1e-16 of a
+// smaller a): for divisors that are densities, volume fractions, wave speeds,
+// determinants or material constants, and dividends that are not a wave's
+// vanishing forerunner; the quotients of velocities keep tdiv.
+__device__ __forceinline__ double qdiv(double a, double b) {
+    const double y = drcp(b);
+    const double q = a * y;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
+}
+__device__ __forceinline__ float qdiv(float a, float b) { return tdiv(a, b); }
+// qdiv in the FP64 form, and correctly rounded in FP32 too (see tdiv_cr)
+__device__ __forceinline__ double qdiv_cr(double a, double b) { return qdiv(a, b); }
+__device__ __forceinline__ float qdiv_cr(float a, float b) { return tdiv_cr(a, b); }
 __device__ __forceinline__ double tsqrt(double x) { return __builtin_sqrt(x); }
 __device__ __forceinline__ float tsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ double tabs(double x) { return __builtin_fabs(x); }
@@ -265,12 +293,12 @@ __device__ inline double pm_tanh(double x) {
     double ax = __builtin_fabs(x);
     if (ax > 20.0) return x > 0.0 ? 1.0 : -1.0;
     double t = pm_expm1(2.0 * ax);
-    double r = t / (t + 2.0);
+    double r = qdiv(t, t + 2.0);
     return x < 0.0 ? -r : r;
 }
 __device__ inline double pm_cosh(double x) {
     double e = pm_exp(__builtin_fabs(x));
-    return (e + 1.0 / e) * 0.5;
+    return (e + qdiv(1.0, e)) * 0.5;
 }
 __device__ inline double pm_rcbrt(double x) {
     uint64_t bits = __builtin_bit_cast(uint64_t, x);
@@ -278,11 +306,11 @@ __device__ inline double pm_rcbrt(double x) {
     double y = __builtin_bit_cast(double, g);
     for (int it = 0; it < 5; ++it) {
         double y3 = (y * y) * y;
-        y = y * ((4.0 - x * y3) / 3.0);
+        y = y * qdiv(4.0 - x * y3, 3.0);
     }
-    double c = 1.0 / y;
-    c = c - (c - x / (c * c)) / 3.0;
-    return 1.0 / c;
+    double c = qdiv(1.0, y);
+    c = c - qdiv(c - qdiv(x, c * c), 3.0);
+    return qdiv(1.0, c);
 }
 
 // log (x = 2^e m, m in [sqrt(2)/2, sqrt(2)), the atanh series of
@@ -309,7 +337,7 @@ __device__ inline double pm_log(double x) {
     const double ln2hi = 6.93147180369123816490e-01;
     const double ln2lo = 1.90821492927058770002e-10;
     const double f = m - 1.0;
-    const double s = f / (2.0 + f);
+    const double s = qdiv(f, 2.0 + f);
     const double z = s * s;
     double q = 2.0 / 25.0;
     q = q * z + 2.0 / 23.0;

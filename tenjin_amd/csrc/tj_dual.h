@@ -32,15 +32,6 @@ struct Dual {
     }
 };
 
-// 1/b for derivative parts: v_rcp_f64's estimate and two Newton steps
-__device__ __forceinline__ double drcp(double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    double e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-b, r, 1.0);
-    return __builtin_fma(r, e, r);
-}
-
 #define TJ_DUAL_FN template <int K> __device__ __forceinline__
 
 TJ_DUAL_FN Dual<K> operator-(const Dual<K>& a) {
@@ -132,6 +123,32 @@ TJ_DUAL_FN Dual<K> tdiv(double a, const Dual<K>& b) {
     return r;
 }
 TJ_DUAL_FN Dual<K> tdiv_cr(const Dual<K>& a, const Dual<K>& b) { return tdiv(a, b); }
+// qdiv: the value and the derivative parts share the divisor's reciprocal
+TJ_DUAL_FN Dual<K> qdiv(const Dual<K>& a, const Dual<K>& b) {
+    Dual<K> r;
+    r.v = qdiv(a.v, b.v);
+    const double rb = drcp(b.v);
+#pragma unroll
+    for (int t = 0; t < K; ++t) r.d[t] = __builtin_fma(-r.v, b.d[t], a.d[t]) * rb;
+    return r;
+}
+TJ_DUAL_FN Dual<K> qdiv(const Dual<K>& a, double b) {
+    Dual<K> r;
+    r.v = qdiv(a.v, b);
+    const double rb = drcp(b);
+#pragma unroll
+    for (int t = 0; t < K; ++t) r.d[t] = a.d[t] * rb;
+    return r;
+}
+TJ_DUAL_FN Dual<K> qdiv(double a, const Dual<K>& b) {
+    Dual<K> r;
+    r.v = qdiv(a, b.v);
+    const double g = -r.v * drcp(b.v);
+#pragma unroll
+    for (int t = 0; t < K; ++t) r.d[t] = g * b.d[t];
+    return r;
+}
+TJ_DUAL_FN Dual<K> qdiv_cr(const Dual<K>& a, const Dual<K>& b) { return qdiv(a, b); }
 TJ_DUAL_FN Dual<K> operator/(const Dual<K>& a, const Dual<K>& b) { return tdiv(a, b); }
 TJ_DUAL_FN Dual<K> operator/(const Dual<K>& a, double b) { return tdiv(a, b); }
 TJ_DUAL_FN Dual<K> operator/(double a, const Dual<K>& b) { return tdiv(a, b); }

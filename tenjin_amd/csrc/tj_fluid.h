@@ -78,7 +78,7 @@ template <typename R>
 __device__ __forceinline__ R vanleer(R r) {
     if (r <= R(0)) return R(0);
     R num = (r < R(1)) ? R(2) * r : R(2);
-    return tdiv(num, R(1) + r);
+    return qdiv(num, R(1) + r);
 }
 template <typename R>
 __device__ __forceinline__ void muscl1(R um, R uc, R up, R& L, R& Rt) {
@@ -108,23 +108,23 @@ __device__ __forceinline__ void muscl(const Prim<NM, Rt>& m_, const Prim<NM, Rt>
 // state in thermal equilibrium.
 template <typename R>
 __device__ __forceinline__ R mix_gamma(const MatT<R>& M, R lam) {
-    return tdiv(lam * M.ga * M.CV + (R(1) - lam) * M.g2 * M.CV2, lam * M.CV + (R(1) - lam) * M.CV2) - R(1);
+    return qdiv(lam * M.ga * M.CV + (R(1) - lam) * M.g2 * M.CV2, lam * M.CV + (R(1) - lam) * M.CV2) - R(1);
 }
 template <typename R>
 __device__ __forceinline__ R mix_rhob(R lam, R rk, R ra) {
-    return tdiv(R(1) - lam, tdiv(R(1), rk) - tdiv(lam, ra));
+    return qdiv(R(1) - lam, qdiv(R(1), rk) - qdiv(lam, ra));
 }
 template <typename R>
 __device__ __forceinline__ void mix_define(const MatT<R>& M, R p, MixV<R>& x) {
-    x.ra = x.rk * (x.lam + (R(1) - x.lam) * tdiv(p - M.pref, p - M.pref2) * tdiv(M.CV2 * M.Gg2, M.CV * M.Gg));
+    x.ra = x.rk * (x.lam + (R(1) - x.lam) * qdiv(p - M.pref, p - M.pref2) * qdiv(M.CV2 * M.Gg2, M.CV * M.Gg));
     x.rb = mix_rhob(x.lam, x.rk, x.ra);
 }
 // mixtureSoundSpeed (equationofstate.cpp:212-226)
 template <typename R>
 __device__ __forceinline__ R mix_c2(const MatT<R>& M, R p, const MixV<R>& x) {
-    R dedrho = (x.lam) * tdiv(M.pref - p, M.Gg * x.rk * x.rk);
-    dedrho += (R(1) - x.lam) * tdiv(M.pref2 - p, M.Gg2 * x.rk * x.rk);
-    return tdiv(tdiv(p, x.rk * x.rk) - dedrho, tdiv(x.lam, x.ra * M.Gg) + tdiv(R(1) - x.lam, x.rb * M.Gg2));
+    R dedrho = (x.lam) * qdiv(M.pref - p, M.Gg * x.rk * x.rk);
+    dedrho += (R(1) - x.lam) * qdiv(M.pref2 - p, M.Gg2 * x.rk * x.rk);
+    return qdiv(qdiv(p, x.rk * x.rk) - dedrho, qdiv(x.lam, x.ra * M.Gg) + qdiv(R(1) - x.lam, x.rb * M.Gg2));
 }
 
 // equationofstate.cpp:37-64 and boxaccesscellarray.cpp:218-252; the mixture
@@ -138,8 +138,8 @@ __device__ __forceinline__ void eos_sums(const Level& lv, const R* a, const R* a
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
         const MatT<R>& M = mat<R>(lv, m);
-        if (MX && m == lv.mixm) G += tdiv(a[m], mix_gamma(M, x.lam));
-        else G += tdiv(a[m], M.Gg);
+        if (MX && m == lv.mixm) G += qdiv(a[m], mix_gamma(M, x.lam));
+        else G += qdiv(a[m], M.Gg);
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
@@ -151,10 +151,10 @@ __device__ __forceinline__ void eos_sums(const Level& lv, const R* a, const R* a
     for (int m = 0; m < NM; ++m) {
         const MatT<R>& M = mat<R>(lv, m);
         if (MX && m == lv.mixm) {
-            const R pa = tdiv(M.pref * a[m], M.Gg), pb = tdiv(M.pref2 * a[m], M.Gg2);
-            Pnt += tdiv(pa * x.lam * x.rk, x.ra) + tdiv(pb * (R(1) - x.lam) * x.rk, x.rb) + R(0);
+            const R pa = qdiv(M.pref * a[m], M.Gg), pb = qdiv(M.pref2 * a[m], M.Gg2);
+            Pnt += qdiv(pa * x.lam * x.rk, x.ra) + qdiv(pb * (R(1) - x.lam) * x.rk, x.rb) + R(0);
         } else {
-            Pnt += tdiv(M.pref * a[m], M.Gg) + R(0) * a[m];
+            Pnt += qdiv(M.pref * a[m], M.Gg) + R(0) * a[m];
         }
     }
 }
@@ -193,13 +193,13 @@ __device__ __forceinline__ void p2c_sound(const Level& lv, const Prim<NM, R>& P,
     for (int m = 0; m < NM; ++m) {
         const MatT<R>& M = mat<R>(lv, m);
         const bool mx = MX && m == lv.mixm;
-        const R c2 = mx ? mix_c2(M, P.p, x) : tdiv(P.p * M.gp1, P.r[m]) - tdiv(M.pref, P.r[m]);
-        const R xi = mx ? tdiv(R(1), mix_gamma(M, x.lam)) : M.xi;
-        a += tmax(R(0), tdiv(xi * c2 * S.ar[m], rho));
+        const R c2 = mx ? mix_c2(M, P.p, x) : qdiv(P.p * M.gp1, P.r[m]) - qdiv(M.pref, P.r[m]);
+        const R xi = mx ? qdiv(R(1), mix_gamma(M, x.lam)) : M.xi;
+        a += tmax(R(0), qdiv(xi * c2 * S.ar[m], rho));
         xt += xi * S.al[m];
     }
     if (a <= R(0)) a = R(1E-6);
-    S.a = tsqrt(tdiv(a, xt));
+    S.a = tsqrt(qdiv(a, xt));
     if (MX && xo) *xo = x;
 }
 
@@ -225,8 +225,8 @@ __device__ __forceinline__ unsigned root_find(const Level& lv, const double* al,
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
         const MatC& Mm = lv.m[m];
-        if (m == lv.mixm) G += al[m] / (mix_gamma(Mm, lam));
-        else G += al[m] / Mm.Gg;
+        if (m == lv.mixm) G += qdiv(al[m], mix_gamma(Mm, lam));
+        else G += qdiv(al[m], Mm.Gg);
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
@@ -238,26 +238,26 @@ __device__ __forceinline__ unsigned root_find(const Level& lv, const double* al,
     for (int m = 0; m < NM; ++m) {
         const MatC& Mm = lv.m[m];
         if (m == lv.mixm) {
-            pal = (Mm.pref * al[m] / Mm.Gg) * lam * x.rk;
-            pbl = (Mm.pref2 * al[m] / Mm.Gg2) * (1.0 - lam) * x.rk;
+            pal = qdiv(Mm.pref * al[m], Mm.Gg) * lam * x.rk;
+            pbl = qdiv(Mm.pref2 * al[m], Mm.Gg2) * (1.0 - lam) * x.rk;
             pconst[m] = 0.0;
         } else {
-            pconst[m] = Mm.pref * al[m] / Mm.Gg + 0.0 * al[m];
+            pconst[m] = qdiv(Mm.pref * al[m], Mm.Gg) + 0.0 * al[m];
         }
     }
     const double cE = E - ke - Ent;
-    const double inv_rk = 1.0 / x.rk;
-    auto rhob = [&](double ra) { return (1.0 - lam) / (inv_rk - lam / ra); };
+    const double inv_rk = qdiv(1.0, x.rk);
+    auto rhob = [&](double ra) { return qdiv(1.0 - lam, inv_rk - qdiv(lam, ra)); };
     auto fn = [&](double ra) {
         const double rb = rhob(ra);
         double Pnt = 0.0;
 #pragma unroll
-        for (int m = 0; m < NM; ++m) Pnt += (m == lv.mixm) ? (pal / (ra) + pbl / (rb) + 0.0) : pconst[m];
-        const double pp = (cE + Pnt) / (G);
-        return ((pp - M.pref) / (ra * M.Gg * M.CV)) - ((pp - M.pref2) / (rb * M.Gg2 * M.CV2));
+        for (int m = 0; m < NM; ++m) Pnt += (m == lv.mixm) ? (qdiv(pal, ra) + qdiv(pbl, rb) + 0.0) : pconst[m];
+        const double pp = qdiv(cE + Pnt, G);
+        return qdiv(pp - M.pref, ra * M.Gg * M.CV) - qdiv(pp - M.pref2, rb * M.Gg2 * M.CV2);
     };
     if (M.pref == 0.0 && M.pref2 == 0.0) {
-        x.ra = x.rk * (lam + (1.0 - lam) * (M.Gg2 * M.CV2) / (M.Gg * M.CV));
+        x.ra = x.rk * (lam + qdiv((1.0 - lam) * (M.Gg2 * M.CV2), M.Gg * M.CV));
         x.rb = mix_rhob(lam, x.rk, x.ra);
         return 0u;
     }
@@ -296,7 +296,7 @@ __device__ __forceinline__ unsigned root_find(const Level& lv, const double* al,
         if (smid == sa) a = mid;  // f(a) keeps its sign: a moves only to a point of that sign
         else b = mid;
         mid = 0.5 * (a + b);
-        if (__builtin_fabs(a - b) / (a + b) < 1E-7 || n >= 2000) {
+        if (qdiv(__builtin_fabs(a - b), a + b) < 1E-7 || n >= 2000) {
             x.ra = mid;
             x.rb = rhob(mid);
             return n >= 2000 ? 64u : 0u;
@@ -314,7 +314,7 @@ __device__ __forceinline__ unsigned c2p(const Level& lv, const double* al, const
     rho = 0.0;
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = ar[m] / al[m];
+        rk[m] = qdiv(ar[m], al[m]);
         rho += ar[m];
     }
     double ke = 0.0;
@@ -330,14 +330,14 @@ __device__ __forceinline__ unsigned c2p(const Level& lv, const double* al, const
         for (int m = 0; m < NM; ++m)
             if (m == lv.mixm) {
                 xm.rk = rk[m];
-                xm.lam = arl / ar[m];
+                xm.lam = qdiv(arl, ar[m]);
             }
         st = root_find<NM>(lv, al, ar, E, ke, xm);
         *x = xm;
     }
     double G, Ent, Pnt;
     eos_sums<NM, double, MX>(lv, al, ar, G, Ent, Pnt, xm);
-    p = (E - ke - Ent + Pnt) / G;
+    p = qdiv(E - ke - Ent + Pnt, G);
     return st;
 }
 
@@ -351,19 +351,24 @@ __device__ __forceinline__ double sound(const Level& lv, const double* al, const
     for (int m = 0; m < NM; ++m) {
         const MatC& M = lv.m[m];
         const bool mx = MX && m == lv.mixm;
-        const double c2 = mx ? mix_c2(M, p, x) : p * M.gp1 / rk[m] - M.pref / rk[m];
-        const double xi = mx ? 1.0 / (mix_gamma(M, x.lam)) : M.xi;
-        a += dmax(0.0, xi * c2 * ar[m] / rho);
+        const double c2 = mx ? mix_c2(M, p, x) : qdiv(p * M.gp1, rk[m]) - qdiv(M.pref, rk[m]);
+        const double xi = mx ? qdiv(1.0, mix_gamma(M, x.lam)) : M.xi;
+        a += dmax(0.0, qdiv(xi * c2 * ar[m], rho));
         xt += xi * al[m];
     }
     if (a <= 0.0) a = 1E-6;
-    return __builtin_sqrt(a / xt);
+    return tsqrt(qdiv(a, xt));
 }
 
 // ------------------------------------------------------------------ HLLC
 // hllc.cpp:5-73 (getSstar, getStarState), 384-487 (calc_fluxes), flux.cpp:5-47.
 // F layout: [0,NM) alpha, [NM,2NM) alphaRho, [2NM,2NM+3) rhoU, 2NM+3 E, 2NM+4 S*.
 // MX: F[2NM+5] is the alpha rho lambda flux (flux.cpp:39, hllc.cpp:26-29).
+// |(S* - u) / S*| < 1e-20 of hllc.cpp:40 without the division: two different
+// floating-point numbers differ by 2^-54 (FP32: 2^-25) of either or more, so
+// the quotient is that small only when they are equal and not 0.
+template <typename R>
+__device__ __forceinline__ bool star_at_speed(R Ss, R u) { return Ss - u == R(0) && Ss != R(0); }
 template <int NM, typename R, bool MX = false>
 __device__ __forceinline__ void hllc(const FSt<NM, R>& L, const FSt<NM, R>& Rs, int d, R* F, R* sa) {
     const FSt<NM, R>& Rr = Rs;
@@ -387,7 +392,7 @@ __device__ __forceinline__ void hllc(const FSt<NM, R>& L, const FSt<NM, R>& Rs, 
     const R SK = useL ? SL : SR;
     const R sigK = useL ? sigL : sigR;
     // star state
-    const R mult = (tabs(tdiv(Ss - K.u[d], Ss)) < R(1E-20)) ? R(1) : tdiv_cr(SK - K.u[d], SK - Ss);
+    const R mult = star_at_speed(Ss, K.u[d]) ? R(1) : qdiv_cr(SK - K.u[d], SK - Ss);
     R arS[NM], rhoS = R(0);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
@@ -398,7 +403,7 @@ __device__ __forceinline__ void hllc(const FSt<NM, R>& L, const FSt<NM, R>& Rs, 
 #pragma unroll
     for (int q = 0; q < 3; ++q) ruS[q] = (q == d) ? mult * K.rho * Ss : mult * ruK[q];
     const R uSd = tdiv(ruS[d], rhoS);
-    const R ES = mult * K.rho * (tdiv(K.E, K.rho) + (Ss - K.u[d]) * (Ss - tdiv(sigK, K.rho * (SK - K.u[d]))));
+    const R ES = mult * K.rho * (qdiv(K.E, K.rho) + (Ss - K.u[d]) * (Ss - qdiv(sigK, K.rho * (SK - K.u[d]))));
     // physical flux of K (flux.cpp:33-47) with sigma = -p I
     R vds = R(0);
 #pragma unroll
@@ -447,7 +452,7 @@ __device__ inline void arec(const Level& lv, const V& U, int i, int j, int k, in
         const R mx = tmax(aL, aR) - mn;
         const R theta = tsgn(aR - aL);
         const R eps = R(1E-20);
-        const R C = (mx < eps) ? R(0) : tdiv(aC - mn + eps, mx + eps);
+        const R C = (mx < eps) ? R(0) : qdiv(aC - mn + eps, mx + eps);
         const R dl = R(1E-4);
         const bool mixed = (C > dl) && (C < (R(0.999999) - dl)) && ((aR - aC) * (aC - aL) >= R(0));
         A.thl[m] = R(0);
@@ -461,13 +466,13 @@ __device__ inline void arec(const Level& lv, const V& U, int i, int j, int k, in
                 const R ny = yny * (a(1, 1) + R(2) * a(0, 1) + a(-1, 1) - a(-1, -1) - R(2) * a(0, -1) - a(1, -1));
                 const R norm = tsqrt(nx * nx + ny * ny);
                 if (norm < R(1E-20)) nvc = R(0);
-                else nvc = (d == 0) ? tabs(tdiv(nx, norm)) : tabs(tdiv(ny, norm));
+                else nvc = (d == 0) ? tabs(qdiv(nx, norm)) : tabs(qdiv(ny, norm));
             }
             const R beta = nvc * R(lv.beta0) + R(0.01);
             const R coshB = tcosh(beta), tanhB = ttanh(beta);
             const R B = texp(theta * beta * ((R(2) * C) - R(1)));
-            const R Ac = tdiv(tdiv(B, coshB) - R(1), tanhB);
-            A.thr[m] = mn + tdiv(mx, R(2)) * (R(1) + theta * tdiv(tanhB + Ac, R(1) + Ac * tanhB));
+            const R Ac = qdiv(qdiv(B, coshB) - R(1), tanhB);
+            A.thr[m] = mn + tdiv(mx, R(2)) * (R(1) + theta * qdiv(tanhB + Ac, R(1) + Ac * tanhB));
             A.thl[m] = mn + tdiv(mx, R(2)) * (R(1) + theta * Ac);
         }
     }
@@ -510,7 +515,7 @@ __device__ __forceinline__ unsigned cleanup_alpha(R* a) {
     }
     if (tot <= R(0)) st |= 8u;
 #pragma unroll
-    for (int m = 0; m < NM; ++m) a[m] *= tdiv(R(1), tot);
+    for (int m = 0; m < NM; ++m) a[m] *= qdiv(R(1), tot);
     return st;
 }
 

@@ -365,7 +365,7 @@ __device__ __forceinline__ void finish_cell(const Level& lv, const MF& Ub, const
             put_state<STAGE == 2>(Uo.at(lv.cs[SOUNDSPEED], i, j, k), a);
             #pragma unroll
             for (int d = 0; d < 3; ++d)  // unrolled: constant indices keep the state in registers
-                if (d < lv.dim) cand = dmin(cand, lv.dx[d] / (a + __builtin_fabs(u[d])));
+                if (d < lv.dim) cand = dmin(cand, qdiv(lv.dx[d], a + __builtin_fabs(u[d])));
         }
     }
 #pragma unroll

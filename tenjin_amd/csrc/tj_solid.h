@@ -41,7 +41,7 @@ __device__ __forceinline__ void inv3(const R* M, R* Mi) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) Mi[i * 3 + j] = tdiv(cof[j * 3 + i], D);
+        for (int j = 0; j < 3; ++j) Mi[i * 3 + j] = qdiv(cof[j * 3 + i], D);
 }
 template <typename R>
 __device__ __forceinline__ void mm3(const R* A, const R* B, R* C) {  // C = A B
@@ -98,8 +98,8 @@ __device__ __forceinline__ void jacobi_spd(const R* Ain, R* a, R* q) {
             // nothing representable, and its reciprocal can overflow
             if (sizeof(R) == 4 && tabs(apq) < R(1e-12) * (tabs(app) + tabs(aqq))) continue;
             const R theta = tdiv(aqq - app, R(2) * apq);
-            const R t = tdiv(theta >= R(0) ? R(1) : R(-1), tabs(theta) + tsqrt(theta * theta + R(1)));
-            const R c = tdiv(R(1), tsqrt(t * t + R(1)));
+            const R t = qdiv(theta >= R(0) ? R(1) : R(-1), tabs(theta) + tsqrt(theta * theta + R(1)));
+            const R c = qdiv(R(1), tsqrt(t * t + R(1)));
             const R s = t * c;
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -181,27 +181,27 @@ __device__ inline void sqrtm_spd(const Dual<K>* Ain, Dual<K>* S) {
 // eta = 1 - rho0/rho, with the Mie-Gruneisen form p = p_H + Gamma rho (e - e_H).
 template <typename R>
 __device__ __forceinline__ R pH(const MatT<R>& M, R rho) {
-    const R eta = R(1) - tdiv(M.rho0, rho);
+    const R eta = R(1) - qdiv(M.rho0, rho);
     const R den = R(1) - M.s * eta;
-    return tdiv(M.rho0 * M.c0 * M.c0 * eta, den * den);
+    return qdiv(M.rho0 * M.c0 * M.c0 * eta, den * den);
 }
 template <typename R>
 __device__ __forceinline__ R eH(const MatT<R>& M, R rho) {
-    const R eta = R(1) - tdiv(M.rho0, rho);
-    return tdiv(pH(M, rho) * eta, R(2) * M.rho0);
+    const R eta = R(1) - qdiv(M.rho0, rho);
+    return qdiv(pH(M, rho) * eta, R(2) * M.rho0);
 }
 template <typename R>
 __device__ __forceinline__ R dpH(const MatT<R>& M, R rho) {
-    const R eta = R(1) - tdiv(M.rho0, rho);
+    const R eta = R(1) - qdiv(M.rho0, rho);
     const R den = R(1) - M.s * eta;
-    const R detadrho = tdiv(M.rho0, rho * rho);
-    return tdiv(M.rho0 * M.c0 * M.c0 * (R(1) + M.s * eta), den * den * den) * detadrho;
+    const R detadrho = qdiv(M.rho0, rho * rho);
+    return qdiv(M.rho0 * M.c0 * M.c0 * (R(1) + M.s * eta), den * den * den) * detadrho;
 }
 template <typename R>
 __device__ __forceinline__ R deH(const MatT<R>& M, R rho) {
-    const R eta = R(1) - tdiv(M.rho0, rho);
-    const R detadrho = tdiv(M.rho0, rho * rho);
-    return tdiv(dpH(M, rho) * eta + pH(M, rho) * detadrho, R(2) * M.rho0);
+    const R eta = R(1) - qdiv(M.rho0, rho);
+    const R detadrho = qdiv(M.rho0, rho * rho);
+    return qdiv(dpH(M, rho) * eta + pH(M, rho) * detadrho, R(2) * M.rho0);
 }
 // componentShearModulus (equationofstate.cpp:77-80, 447-450, 548-551): G0 of
 // the Us-up and Wilkins solids, G0 (rho_k/rho0)^(beta + 1) of the Romenskii
@@ -213,7 +213,7 @@ template <bool RW, typename R>
 __device__ __forceinline__ R shearG(const MatT<R>& M, R rk) {
     if (M.eos == 1 || M.eos == 3) return M.G0;
     if constexpr (RW) {
-        if (M.eos == 2) return M.G0 * tpow(tdiv(rk, M.rho0), M.eb + R(1.0));
+        if (M.eos == 2) return M.G0 * tpow(qdiv(rk, M.rho0), M.eb + R(1.0));
     }
     return R(0);
 }
@@ -223,37 +223,37 @@ __device__ __forceinline__ R shearG(const MatT<R>& M, R rk) {
 // dp_s/drho of material M at density rk; a = alpha, ar = alpha rho.
 template <typename R>
 __device__ __forceinline__ R cold_e(const MatT<R>& M, R ar, R rk) {
-    const R x = tdiv(rk, M.rho0);
+    const R x = qdiv(rk, M.rho0);
     if (M.eos == 2) {
         const R xa = tpow(x, M.ea);
-        return ar * (tdiv(M.K0, R(2.0) * M.rho0 * M.ea * M.ea) * (xa - R(1.0)) * (xa - R(1.0)));
+        return ar * (qdiv(M.K0, R(2.0) * M.rho0 * M.ea * M.ea) * (xa - R(1.0)) * (xa - R(1.0)));
     }
-    return ar * tdiv(M.e1 + M.e2 * x * x + M.e3 * x + tdiv(M.e4, x) - M.e5 * tlog(x), M.rho0);
+    return ar * qdiv(M.e1 + M.e2 * x * x + M.e3 * x + qdiv(M.e4, x) - M.e5 * tlog(x), M.rho0);
 }
 template <typename R>
 __device__ __forceinline__ R cold_p(const MatT<R>& M, R a, R rk) {
-    const R x = tdiv(rk, M.rho0);
-    if (M.eos == 2) return tdiv(a, M.Gg) * (tdiv(M.K0, M.ea) * tpow(x, M.ea + R(1.0)) * (tpow(x, M.ea) - R(1.0)));
-    return tdiv(a, M.Gg) * ((R(2.0) * M.e2 * x * x * x + M.e3 * x * x - M.e4 - M.e5 * x));
+    const R x = qdiv(rk, M.rho0);
+    if (M.eos == 2) return qdiv(a, M.Gg) * (qdiv(M.K0, M.ea) * tpow(x, M.ea + R(1.0)) * (tpow(x, M.ea) - R(1.0)));
+    return qdiv(a, M.Gg) * ((R(2.0) * M.e2 * x * x * x + M.e3 * x * x - M.e4 - M.e5 * x));
 }
 template <typename R>
 __device__ __forceinline__ R dGdrho(const MatT<R>& M, R rk) {
-    if (M.eos == 2) return tdiv(M.G0 * (M.eb + R(1.0)) * tpow(tdiv(rk, M.rho0), M.eb), M.rho0);
+    if (M.eos == 2) return qdiv(M.G0 * (M.eb + R(1.0)) * tpow(qdiv(rk, M.rho0), M.eb), M.rho0);
     return R(0.0);
 }
 template <typename R>
 __device__ __forceinline__ R dG2drho2(const MatT<R>& M, R rk) {
-    if (M.eos == 2) return tdiv(M.G0 * (M.eb + R(1.0)) * (M.eb) * tpow(tdiv(rk, M.rho0), M.eb - R(1.0)), M.rho0 * M.rho0);
+    if (M.eos == 2) return qdiv(M.G0 * (M.eb + R(1.0)) * (M.eb) * tpow(qdiv(rk, M.rho0), M.eb - R(1.0)), M.rho0 * M.rho0);
     return R(0.0);
 }
 template <typename R>
 __device__ __forceinline__ R dpc_drho(const MatT<R>& M, R rk) {
-    const R x = tdiv(rk, M.rho0);
+    const R x = qdiv(rk, M.rho0);
     if (M.eos == 2) {
         const R xa = tpow(x, M.ea);
-        return tdiv(M.K0, M.ea * M.rho0) * xa * ((R(2.0) * M.ea + R(1.0)) * xa - (M.ea + R(1.0)));
+        return qdiv(M.K0, M.ea * M.rho0) * xa * ((R(2.0) * M.ea + R(1.0)) * xa - (M.ea + R(1.0)));
     }
-    return tdiv(R(6.0) * M.e2 * x * x + R(2.0) * M.e3 * x - M.e5, M.rho0);
+    return qdiv(R(6.0) * M.e2 * x * x + R(2.0) * M.e3 * x - M.e5, M.rho0);
 }
 
 // coldCompressionInternalEnergy + shearInternalEnergy and coldCompressionPressure
@@ -271,7 +271,7 @@ __device__ __forceinline__ R rw_pressure(const MatT<R>& M, R a, R rk, R hj2) {
     if constexpr (!RW) {
         return R(0);
     } else {
-        return cold_p(M, a, rk) + tdiv(a, M.Gg) * ((rk * dGdrho(M, rk) - shearG<true>(M, rk)) * hj2);
+        return cold_p(M, a, rk) + qdiv(a, M.Gg) * ((rk * dGdrho(M, rk) - shearG<true>(M, rk)) * hj2);
     }
 }
 // getSoundSpeedContribution of a Romenskii or Wilkins material
@@ -283,9 +283,9 @@ __device__ __forceinline__ R rw_c2(const MatT<R>& M, R p, R a, R rk, R hj2) {
         return R(0);
     } else {
         const R G = shearG<true>(M, rk);
-        const R ps = tdiv(a, M.Gg) * ((rk * dGdrho(M, rk) - G) * hj2);
-        return tdiv(p * (M.Gg + R(1.0)) - (cold_p(M, a, rk) + ps) * (M.Gg + R(1.0)), rk) + dpc_drho(M, rk) +
-               rk * dG2drho2(M, rk) * hj2 + tdiv((R(4.0) / R(3.0)) * G, rk);
+        const R ps = qdiv(a, M.Gg) * ((rk * dGdrho(M, rk) - G) * hj2);
+        return qdiv(p * (M.Gg + R(1.0)) - (cold_p(M, a, rk) + ps) * (M.Gg + R(1.0)), rk) + dpc_drho(M, rk) +
+               rk * dG2drho2(M, rk) * hj2 + qdiv((R(4.0) / R(3.0)) * G, rk);
     }
 }
 
@@ -297,7 +297,7 @@ __device__ __forceinline__ void eos_sums_s(const Level& lv, const R* a, const R*
     Ent = R(0);
     Pnt = R(0);
 #pragma unroll
-    for (int m = 0; m < NM; ++m) G += tdiv(a[m], mat<R>(lv, m).Gg);
+    for (int m = 0; m < NM; ++m) G += qdiv(a[m], mat<R>(lv, m).Gg);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
         const MatT<R>& M = mat<R>(lv, m);
@@ -309,10 +309,10 @@ __device__ __forceinline__ void eos_sums_s(const Level& lv, const R* a, const R*
     for (int m = 0; m < NM; ++m) {
         const MatT<R>& M = mat<R>(lv, m);
         if (M.eos == 1)
-            Pnt += tdiv(a[m], M.Gg) * pH(M, rk[m]) + tdiv(a[m], M.Gg) * ((rk[m] * R(0) - shearG<RW>(M, rk[m])) * hj2);
+            Pnt += qdiv(a[m], M.Gg) * pH(M, rk[m]) + qdiv(a[m], M.Gg) * ((rk[m] * R(0) - shearG<RW>(M, rk[m])) * hj2);
         else if (RW && M.eos >= 2)
             Pnt += rw_pressure<RW>(M, a[m], rk[m], hj2);
-        else Pnt += tdiv(M.pref * a[m], M.Gg) + R(0) * a[m];
+        else Pnt += qdiv(M.pref * a[m], M.Gg) + R(0) * a[m];
     }
 }
 // getSoundSpeedContribution: stiffened gas (equationofstate.cpp:61-64), the
@@ -322,10 +322,10 @@ __device__ __forceinline__ void eos_sums_s(const Level& lv, const R* a, const R*
 template <bool RW, typename R>
 __device__ __forceinline__ R c2_s(const MatT<R>& M, R p, R a, R rk, R hj2) {
     if (M.eos == 1)
-        return tdiv(p * M.gp1 - pH(M, rk) + M.gp1 * M.G0 * hj2, rk) + dpH(M, rk) - M.Gg * rk * deH(M, rk) +
-               tdiv((R(4.0) / R(3.0)) * M.G0, rk);
+        return qdiv(p * M.gp1 - pH(M, rk) + M.gp1 * M.G0 * hj2, rk) + dpH(M, rk) - M.Gg * rk * deH(M, rk) +
+               qdiv((R(4.0) / R(3.0)) * M.G0, rk);
     if (RW && M.eos >= 2) return rw_c2<RW>(M, p, a, rk, hj2);
-    return tdiv(p * M.gp1, rk) - tdiv(M.pref, rk);
+    return qdiv(p * M.gp1, rk) - qdiv(M.pref, rk);
 }
 template <int NM, bool RW, typename R>
 __device__ __forceinline__ R sound_s(const Level& lv, const R* al, const R* ar, const R* rk, R rho, R p, R hj2) {
@@ -333,11 +333,11 @@ __device__ __forceinline__ R sound_s(const Level& lv, const R* al, const R* ar, 
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
         const MatT<R>& M = mat<R>(lv, m);
-        a += tmax(R(0), tdiv(M.xi * c2_s<RW>(M, p, al[m], rk[m], hj2) * ar[m], rho));
+        a += tmax(R(0), qdiv(M.xi * c2_s<RW>(M, p, al[m], rk[m], hj2) * ar[m], rho));
         xt += M.xi * al[m];
     }
     if (a <= R(0)) a = R(1E-6);
-    return tsqrt(tdiv(a, xt));
+    return tsqrt(qdiv(a, xt));
 }
 // stressTensor column d (boxaccesscellarray.cpp:176-216)
 template <int NM, bool RW, typename R>
@@ -348,11 +348,11 @@ __device__ __forceinline__ void stress_col(const Level& lv, const R* al, const R
     for (int m = 0; m < NM; ++m)
         if (mat<R>(lv, m).solid) {
             solid = 1;
-            Gt += shearG<RW>(mat<R>(lv, m), rk[m]) * tdiv(al[m], mat<R>(lv, m).Gg);
+            Gt += shearG<RW>(mat<R>(lv, m), rk[m]) * qdiv(al[m], mat<R>(lv, m).Gg);
         }
 #pragma unroll
-    for (int m = 0; m < NM; ++m) Gi += tdiv(al[m], mat<R>(lv, m).Gg);
-    Gt = tdiv(Gt, Gi);
+    for (int m = 0; m < NM; ++m) Gi += qdiv(al[m], mat<R>(lv, m).Gg);
+    Gt = qdiv(Gt, Gi);
 #pragma unroll
     for (int r = 0; r < 3; ++r)
         sig[r] = solid ? -p * (r == d ? R(1) : R(0)) + R(2) * Gt * dH[r * 3 + d] : -p * (r == d ? R(1) : R(0));
@@ -441,8 +441,8 @@ template <int NM, typename R>
 __device__ __forceinline__ void c2p_rk_e(const Level& lv, const R* al, const R* ar, const R* are, R* rk, R* e) {
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = tdiv(ar[m], al[m]);
-        e[m] = mat<R>(lv, m).plastic ? tdiv(are[m], ar[m]) : R(0);
+        rk[m] = qdiv(ar[m], al[m]);
+        e[m] = mat<R>(lv, m).plastic ? qdiv(are[m], ar[m]) : R(0);
     }
 }
 
@@ -454,9 +454,9 @@ __device__ __forceinline__ R c2p_s(const Level& lv, const R* al, const R* ar, co
     rho = R(0);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = tdiv(ar[m], al[m]);
+        rk[m] = qdiv(ar[m], al[m]);
         rho += ar[m];
-        e[m] = mat<R>(lv, m).plastic ? tdiv(are[m], ar[m]) : R(0);
+        e[m] = mat<R>(lv, m).plastic ? qdiv(are[m], ar[m]) : R(0);
     }
     const R hj2 = hencky(V, dH);
     R ke = R(0);
@@ -467,7 +467,7 @@ __device__ __forceinline__ R c2p_s(const Level& lv, const R* al, const R* ar, co
     }
     R G, Ent, Pnt;
     eos_sums_s<NM, RW, R>(lv, al, ar, rk, hj2, G, Ent, Pnt);
-    p = tdiv(E - ke - Ent + Pnt, G);
+    p = qdiv(E - ke - Ent + Pnt, G);
     return hj2;
 }
 
@@ -477,11 +477,11 @@ __device__ __forceinline__ R transverse(const Level& lv, const R* al, const R* r
     R b = R(0), g = R(0);
 #pragma unroll
     for (int m = 0; m < NM; ++m)
-        if (mat<R>(lv, m).solid) b += tdiv(tdiv(al[m], mat<R>(lv, m).Gg) * shearG<RW>(mat<R>(lv, m), rk[m]), rk[m]);
+        if (mat<R>(lv, m).solid) b += qdiv(qdiv(al[m], mat<R>(lv, m).Gg) * shearG<RW>(mat<R>(lv, m), rk[m]), rk[m]);
     if (tisnan(b) || b < R(0)) b = R(0);
 #pragma unroll
-    for (int m = 0; m < NM; ++m) g += tdiv(al[m], mat<R>(lv, m).Gg);
-    R t = tsqrt(tdiv(b, g));
+    for (int m = 0; m < NM; ++m) g += qdiv(al[m], mat<R>(lv, m).Gg);
+    R t = tsqrt(qdiv(b, g));
     if (tisnan(t)) t = R(0);
     return t;
 }
@@ -495,13 +495,13 @@ struct SStar {
 template <int NM, typename R>
 __device__ __forceinline__ void star_s(const Level& lv, const SSt<NM, R>& K, const R* ruK, R SK, R Ss, int d,
                                        SStar<NM, R>& T) {
-    const R mult = (tabs(tdiv(Ss - K.u[d], Ss)) < R(1E-20)) ? R(1) : tdiv_cr(SK - K.u[d], SK - Ss);
+    const R mult = star_at_speed(Ss, K.u[d]) ? R(1) : qdiv_cr(SK - K.u[d], SK - Ss);
     T.rho = R(0);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
         T.al[m] = K.al[m];
         T.ar[m] = mult * K.ar[m];
-        T.rk[m] = tdiv(T.ar[m], T.al[m]);
+        T.rk[m] = qdiv(T.ar[m], T.al[m]);
         T.are[m] = mat<R>(lv, m).plastic ? mult * K.are[m] : R(0);
         T.rho += T.ar[m];
     }
@@ -512,7 +512,7 @@ __device__ __forceinline__ void star_s(const Level& lv, const SSt<NM, R>& K, con
 #pragma unroll
         for (int c = 0; c < 3; ++c) T.V[r * 3 + c] = (r == d) ? K.V[r * 3 + c] : mult * K.V[r * 3 + c];
     }
-    T.E = mult * K.rho * (tdiv(K.E, K.rho) + (Ss - K.u[d]) * (Ss - tdiv(K.sig[d], K.rho * (SK - K.u[d]))));
+    T.E = mult * K.rho * (qdiv(K.E, K.rho) + (Ss - K.u[d]) * (Ss - qdiv(K.sig[d], K.rho * (SK - K.u[d]))));
 }
 
 // conservative-variable vector of a state (order of the flux layout):
@@ -648,7 +648,7 @@ __device__ inline void wave5(const Level& lv, const SSt<NM, Rt>& L, const SSt<NM
         const Rt aL = Ls.rho * (Ss - SLT), aR = Rs.rho * (Ss - SRT);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-            sigS[i] = tdiv(Ls.rho * (Ss - SLT) * Rs.rho * (Ss - SRT) * (L.u[i] - R.u[i]) + Ls.rho * (Ss - SLT) * R.sig[i] -
+            sigS[i] = qdiv(Ls.rho * (Ss - SLT) * Rs.rho * (Ss - SRT) * (L.u[i] - R.u[i]) + Ls.rho * (Ss - SLT) * R.sig[i] -
                                Rs.rho * (Ss - SRT) * L.sig[i],
                            aL - aR);
         Rt uss[NC];
@@ -658,16 +658,16 @@ __device__ inline void wave5(const Level& lv, const SSt<NM, Rt>& L, const SSt<NM
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             if (r == d) continue;
-            uss[2 * NM + r] += tdiv(sigS[r] - K.sig[r], Ss - SKT);
+            uss[2 * NM + r] += qdiv(sigS[r] - K.sig[r], Ss - SKT);
             ussu[r] = tdiv(uss[2 * NM + r], Ks.rho);
         }
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             if (r == d) continue;
-            uss[2 * NM + 3] += tdiv(ussu[r] * sigS[r] - K.u[r] * K.sig[r], Ss - SKT);
+            uss[2 * NM + 3] += qdiv(ussu[r] * sigS[r] - K.u[r] * K.sig[r], Ss - SKT);
 #pragma unroll
             for (int c = 0; c < 3; ++c)
-                uss[2 * NM + 4 + r * 3 + c] += tdiv(uss[2 * NM + 4 + d * 3 + c] * (ussu[r] - K.u[r]), Ss - SKT);
+                uss[2 * NM + 4 + r * 3 + c] += qdiv(uss[2 * NM + 4 + d * 3 + c] * (ussu[r] - K.u[r]), Ss - SKT);
         }
 #pragma unroll
         for (int n = NM; n < NC; ++n) F[n] = f[n] + SK * (uS[n] - uK[n]) + SKT * (uss[n] - uS[n]);
@@ -704,7 +704,7 @@ __device__ inline unsigned plastic_cell(const Level& lv, const R* al, const R* a
         R J, Jn;
         if (M.solid) {
             J = tsqrt(hj2);
-            if (shearG<RW>(M, rk[m]) * J * s3 > M.yield) Jn = tdiv(M.yield, s3 * shearG<RW>(M, rk[m]));
+            if (shearG<RW>(M, rk[m]) * J * s3 > M.yield) Jn = qdiv(M.yield, s3 * shearG<RW>(M, rk[m]));
             else Jn = J;
             e[m] += s23 * (J - Jn);
             are[m] = e[m] * ar[m];
@@ -714,12 +714,12 @@ __device__ inline unsigned plastic_cell(const Level& lv, const R* al, const R* a
             e[m] = R(0);
             are[m] = R(0);
         }
-        JB += tdiv(al[m], M.Gg) * J;
-        JT += tdiv(al[m], M.Gg) * Jn;
-        norm += tdiv(al[m], M.Gg);
+        JB += qdiv(al[m], M.Gg) * J;
+        JT += qdiv(al[m], M.Gg) * Jn;
+        norm += qdiv(al[m], M.Gg);
     }
-    JB *= tdiv(R(1), norm);
-    JT *= tdiv(R(1), norm);
+    JB *= qdiv(R(1), norm);
+    JT *= qdiv(R(1), norm);
     if (JB == 0.0 && JT == 0.0) {
         JB = R(1);
         JT = R(1);
@@ -730,7 +730,7 @@ __device__ inline unsigned plastic_cell(const Level& lv, const R* al, const R* a
     for (int q = 0; q < 9; ++q) {
         const double dl = (q / 3 == q % 3) ? 1.0 : 0.0;
         if (dH[q] != 0.0 && JB == 0.0 && JT != 0.0) st |= 16u;
-        else dH[q] *= tdiv(JT, JB);
+        else dH[q] *= qdiv(JT, JB);
         t1[q] = dl + 0.5 * dH[q];
         t2[q] = dl - 0.5 * dH[q];
     }
@@ -761,7 +761,7 @@ __device__ inline void cleanup_v(const Level& lv, const S* al, S* V) {
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
         const R dl = (q / 3 == q % 3) ? R(1) : R(0);
-        V[q] = (S)tdiv((Sq[q] * norm * tsd) + dl * (ta - tsd), ta);
+        V[q] = (S)qdiv((Sq[q] * norm * tsd) + dl * (ta - tsd), ta);
     }
 }
 

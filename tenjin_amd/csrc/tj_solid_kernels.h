@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256) void k_update_s(Level lv, MF Uin, MF Ub, MF Uo
                 put_state<STAGE == 2>(Uo.at(lv.cs[SOUNDSPEED], i, j, k), a);
                 #pragma unroll
                 for (int d = 0; d < 3; ++d)  // unrolled: constant indices keep the state in registers
-                    if (d < lv.dim) cand = dmin(cand, lv.dx[d] / (a + __builtin_fabs(C.u[d])));
+                    if (d < lv.dim) cand = dmin(cand, qdiv(lv.dx[d], a + __builtin_fabs(C.u[d])));
             }
         }
         store_scell<NM, STAGE == 2>(lv, Uo, i, j, k, C);
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(256) void k_sound_dt_s(Level lv, MF U, Clock* clk) 
         U.at(lv.cs[SOUNDSPEED], i, j, k) = a;
         #pragma unroll
         for (int d = 0; d < 3; ++d)  // unrolled: constant indices keep the state in registers
-            if (d < lv.dim) cand = dmin(cand, lv.dx[d] / (a + __builtin_fabs(C.u[d])));
+            if (d < lv.dim) cand = dmin(cand, qdiv(lv.dx[d], a + __builtin_fabs(C.u[d])));
     }
     block_min_to(cand, dt_slot(lv, clk));
 }
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(256) void k_post_s(Level lv, MF U, Clock* clk, unsi
             U.at(lv.cs[SOUNDSPEED], i, j, k) = a;
             #pragma unroll
             for (int d = 0; d < 3; ++d)  // unrolled: constant indices keep the state in registers
-                if (d < lv.dim) cand = dmin(cand, lv.dx[d] / (a + __builtin_fabs(C.u[d])));
+                if (d < lv.dim) cand = dmin(cand, qdiv(lv.dx[d], a + __builtin_fabs(C.u[d])));
         }
         store_scell<NM>(lv, U, i, j, k, C);
     }

@@ -424,7 +424,7 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
             const R mx = tmax(aL, aR) - mn;
             const R theta = tsgn(aR - aL);
             const R eps = R(1E-20);
-            const R Cq = (mx < eps) ? R(0) : tdiv(aC - mn + eps, mx + eps);
+            const R Cq = (mx < eps) ? R(0) : qdiv(aC - mn + eps, mx + eps);
             const R dl = R(1E-4);
             const bool mixed = (Cq > dl) && (Cq < (R(0.999999) - dl)) && ((aR - aC) * (aC - aL) >= R(0));
             A.thl[m] = R(0);
@@ -435,12 +435,12 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
                 const R nxv = ynx * (a(1, 1) + R(2) * a(1, 0) + a(1, -1) - a(-1, 1) - R(2) * a(-1, 0) - a(-1, -1));
                 const R nyv = yny * (a(1, 1) + R(2) * a(0, 1) + a(-1, 1) - a(-1, -1) - R(2) * a(0, -1) - a(1, -1));
                 const R norm = tsqrt(nxv * nxv + nyv * nyv);
-                const R nvc = (norm < R(1E-20)) ? R(0) : tabs(tdiv(nyv, norm));
+                const R nvc = (norm < R(1E-20)) ? R(0) : tabs(qdiv(nyv, norm));
                 const R beta = nvc * R(lv.beta0) + R(0.01);
                 const R coshB = tcosh(beta), tanhB = ttanh(beta);
                 const R B = texp(theta * beta * ((R(2) * Cq) - R(1)));
-                const R Ac = tdiv(tdiv(B, coshB) - R(1), tanhB);
-                A.thr[m] = mn + tdiv(mx, R(2)) * (R(1) + theta * tdiv(tanhB + Ac, R(1) + Ac * tanhB));
+                const R Ac = qdiv(qdiv(B, coshB) - R(1), tanhB);
+                A.thr[m] = mn + tdiv(mx, R(2)) * (R(1) + theta * qdiv(tanhB + Ac, R(1) + Ac * tanhB));
                 A.thl[m] = mn + tdiv(mx, R(2)) * (R(1) + theta * Ac);
             }
         }

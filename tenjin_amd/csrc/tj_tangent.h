@@ -216,7 +216,7 @@ __device__ __forceinline__ double tsound_cand(const Level& lv, const DMF<K>& U, 
     T c = T(__builtin_huge_val());
 #pragma unroll
     for (int d = 0; d < 3; ++d)
-        if (d < lv.dim) c = tmin(c, tdiv(lv.dx[d], a + tabs(C.u[d])));
+        if (d < lv.dim) c = tmin(c, qdiv(lv.dx[d], a + tabs(C.u[d])));
     const long long nc = lv.ncells;
     cand[id] = c.v;
 #pragma unroll
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(256) void k_tinit_p2c_s(Level lv, DMF<K> U, int shi
 #pragma unroll
         for (int m = 0; m < NM; ++m) ar[m] = P.a[m] * P.r[m];
         eos_sums_s<NM, false, T>(lv, P.a, ar, P.r, U.get(lv.cs[HJ2], i, j, k), G, Ent, Pnt);
-        P.p += tdiv(Pnt, G);
+        P.p += qdiv(Pnt, G);
         U.put(lv.cs[PRESSURE], i, j, k, P.p);
     }
     SSt<NM, T> S;
@@ -707,7 +707,7 @@ __device__ __forceinline__ void tc2p_f(const Level& lv, const Dual<K>* al, const
     rho = T(0.0);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = tdiv(ar[m], al[m]);
+        rk[m] = qdiv(ar[m], al[m]);
         rho += ar[m];
     }
     T ke = T(0.0);
@@ -718,7 +718,7 @@ __device__ __forceinline__ void tc2p_f(const Level& lv, const Dual<K>* al, const
     }
     T G, Ent, Pnt;
     eos_sums<NM, T>(lv, al, ar, G, Ent, Pnt);
-    p = tdiv(E - ke - Ent + Pnt, G);
+    p = qdiv(E - ke - Ent + Pnt, G);
 }
 // getSoundSpeed (sound of tj_fluid.h, no mixture) on dual numbers
 template <int NM, int K>
@@ -729,12 +729,12 @@ __device__ __forceinline__ Dual<K> tsound_f(const Level& lv, const Dual<K>* al, 
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
         const MatT<T>& M = mat<T>(lv, m);
-        const T c2 = tdiv(p * M.gp1, rk[m]) - tdiv(M.pref, rk[m]);
-        a += tmax(T(0.0), tdiv(M.xi * c2 * ar[m], rho));
+        const T c2 = qdiv(p * M.gp1, rk[m]) - qdiv(M.pref, rk[m]);
+        a += tmax(T(0.0), qdiv(M.xi * c2 * ar[m], rho));
         xt += M.xi * al[m];
     }
     if (a <= 0.0) a = T(1E-6);
-    return tsqrt(tdiv(a, xt));
+    return tsqrt(qdiv(a, xt));
 }
 template <int NM, int K>
 __device__ __forceinline__ double tcand_f(const Level& lv, const DMF<K>& U, Dual<K> a, const Dual<K>* u, int i, int j,
@@ -744,7 +744,7 @@ __device__ __forceinline__ double tcand_f(const Level& lv, const DMF<K>& U, Dual
     T c = T(__builtin_huge_val());
 #pragma unroll
     for (int d = 0; d < 3; ++d)
-        if (d < lv.dim) c = tmin(c, tdiv(lv.dx[d], a + tabs(u[d])));
+        if (d < lv.dim) c = tmin(c, qdiv(lv.dx[d], a + tabs(u[d])));
     const long long nc = lv.ncells;
     cand[id] = c.v;
 #pragma unroll
@@ -906,7 +906,7 @@ __global__ __launch_bounds__(256) void k_tinit_p2c_f(Level lv, DMF<K> U, int shi
 #pragma unroll
         for (int m = 0; m < NM; ++m) ar[m] = P.a[m] * P.r[m];
         eos_sums<NM, T>(lv, P.a, ar, G, Ent, Pnt);
-        P.p += tdiv(Pnt, G);
+        P.p += qdiv(Pnt, G);
         U.put(lv.cs[PRESSURE], i, j, k, P.p);
     }
     FSt<NM, T> S;
