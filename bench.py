@@ -76,6 +76,17 @@ FLUID_KERNEL_BYTES = {
 # two-material fluid with one mixture material: 9 primitives (lambda), 10
 # flux comps (alpha rho lambda), 19 persistent comps written by the update
 MIX_KERNEL_BYTES = {
+    # stage kernels: 9 primitives + 7 further conserved comps in, the partial
+    # state (9) and 2 star alphas out; y as above, in stage 2 also base and
+    # sound speed
+    "xstage1": 128 + 72 + 16,
+    "xstage2": 128 + 72 + 16,
+    "ystage1": 72 + 72 + 16 + 152,
+    "ystage2_post": 72 + 72 + 16 + 152 + 152 + 8,
+    "xstage1_mixed": 128 + 72 + 16,
+    "xstage2_mixed": 128 + 72 + 16,
+    "ystage1_mixed": 72 + 72 + 16 + 152,
+    "ystage2_post_mixed": 72 + 72 + 16 + 152 + 152 + 8,
     "flux_x": 72 + 80 + 16,
     "flux_y": 72 + 80 + 16,
     "update_stage1": 72 + 2 * 80 + 152,
@@ -86,28 +97,33 @@ MIX_KERNEL_BYTES = {
     "update_stage2_post_mixed": 72 + 2 * 40 + 152 + 152 + 8,
 }
 SOLID_KERNEL_BYTES = {
-    # 19 primitives in (alpha, rho_k, epsilon, u, p, V), 23 face comps out
-    # (19 conserved fluxes, S*, the V* row of the face)
-    "flux_x": 152 + 184,
-    "flux_y": 152 + 184,
-    "flux_z": 152 + 184,
-    # 19 conserved in, 3 directions x 23 face comps, 29 state comps out
-    "update_stage1": 152 + 3 * 184 + 232,
+    # 19 primitives in (alpha, rho_k, epsilon, u, p, V), 20 face comps out
+    # (16 conserved fluxes, the row of V along the pass having none, S*, the
+    # V* row of the face)
+    "flux_x": 152 + 160,
+    "flux_y": 152 + 160,
+    "flux_z": 152 + 160,
+    # 19 conserved in, 3 directions x 20 face comps, 29 state comps out
+    "update_stage1": 152 + 3 * 160 + 232,
+    # the y pass and stage 1's update in one launch: 19 primitives and 8 further
+    # conserved comps in, the other directions' face comps, 29 comps out
+    "flux_y_update1": 152 + 64 + 2 * 160 + 232,
     # + 29 base comps in (RK average), + sound speed out
-    "update_stage2_post": 152 + 3 * 184 + 232 + 232 + 8,
-    # mixed form: FP32 flux planes (23 comps x 4 B), FP64 state
-    "flux_x_mixed": 152 + 92,
-    "flux_y_mixed": 152 + 92,
-    "flux_z_mixed": 152 + 92,
-    "update_stage1_mixed": 152 + 3 * 92 + 232,
-    "update_stage2_post_mixed": 152 + 3 * 92 + 232 + 232 + 8,
+    "update_stage2_post": 152 + 3 * 160 + 232 + 232 + 8,
+    # mixed form: FP32 flux planes (20 comps x 4 B), FP64 state
+    "flux_x_mixed": 152 + 80,
+    "flux_y_mixed": 152 + 80,
+    "flux_z_mixed": 152 + 80,
+    "update_stage1_mixed": 152 + 3 * 80 + 232,
+    "flux_y_update1_mixed": 152 + 64 + 2 * 80 + 232,
+    "update_stage2_post_mixed": 152 + 3 * 80 + 232 + 232 + 8,
 }
 # 8 (3 N_s + 2 N_c): N_s/N_c = 14/8 (two-material fluid), 27/19 (two-material solid)
 # reactive2d: N_s = 14 + 4 (alpha rho lambda, lambda, two phase densities), N_c = 9
 # stage forms of tj_set_tuning's fuse argument, and the workloads whose levels
-# the stage kernels serve (2D fluid, no mixture)
+# the stage kernels serve (2D fluid)
 FORMS = {"stage": 2, "planes": 0, "march": 1}
-STAGE2D_WORKLOADS = ("inclusion2d", "explosion_rz")
+STAGE2D_WORKLOADS = ("inclusion2d", "explosion_rz", "reactive2d")
 
 STEP_BYTES = {"inclusion2d": 464, "plate3d": 952, "tube1d": 464, "ensemble": 464, "explosion_rz": 464,
               "reactive2d": 8 * (3 * 18 + 2 * 9)}

@@ -163,12 +163,13 @@ int tj_bind_level(tj_ctx* ctx, const tj_level_desc* desc);
 /* Tuning: rows per marching segment of the y/z flux passes (seglen > 0
  * fixes it; 0, the default, picks it per pass from the level's shape and the
  * kernel's occupancy so that the segments fill the device's wave slots
- * evenly), and the form of an RK stage of a fluid level:
- *   fuse = 2 (default): on two-dimensional levels without a mixture, the
- *            stage kernels -- the x pass with the x part of the update, then
- *            the y pass over LDS tiles with the rest of the update -- and no
- *            flux planes; other levels as fuse = 0;
- *   fuse = 1: flux planes, the update inside the last directional pass;
+ * evenly), and the form of an RK stage:
+ *   fuse = 2 (default): on two-dimensional fluid levels, the stage kernels --
+ *            the x pass with the x part of the update, then the y pass over
+ *            LDS tiles with the rest of the update -- and no flux planes; on
+ *            Us-up solid levels the y pass and stage 1's update in one launch;
+ *            other levels as fuse = 0;
+ *   fuse = 1: flux planes, the update inside a fluid level's last pass;
  *   fuse = 0: flux planes and an update kernel of its own.
  * Every choice gives identical results; a value < 0 leaves that setting
  * unchanged. */

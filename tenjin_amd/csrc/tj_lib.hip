@@ -437,7 +437,7 @@ int tj_bind_level(tj_ctx* c, const tj_level_desc* d) {
         HIPCHK(c, hipMemcpy(c->d_edge[a], fl.data(), fl.size(), hipMemcpyHostToDevice));
         lv.edge[a] = c->d_edge[a];
     }
-    c->nfc = d->SOLID ? 3 * d->nmat + 17 : 2 * d->nmat + 5 + (lv.mixm >= 0 ? 1 : 0);
+    c->nfc = d->SOLID ? 3 * d->nmat + 14 : 2 * d->nmat + 5 + (lv.mixm >= 0 ? 1 : 0);
     for (int a = 0; a < d->dim; ++a) {
         Faces& F = c->F[a];
         F.nx = lv.n[0] + (a == 0);
@@ -781,6 +781,26 @@ static void launch_pass_solid(tj_ctx* c, const MF& Uin, int d, const FacesT<R>* 
         launch_solid_yz<R, RW, 2>(c, Uin, F[2]);
     }
 }
+// Stage 1 with the y pass and the update in one launch, after the other
+// passes (Us-up and fluid materials).
+template <typename R>
+static void launch_stage1_solid_t(tj_ctx* c, const MF& in, const MF& out, const FacesT<R>* F) {
+    static const char* names[2][3] = {{"flux_x", "flux_y_update1", "flux_z"},
+                                      {"flux_x_mixed", "flux_y_update1_mixed", "flux_z_mixed"}};
+    const int mixed = sizeof(R) == 4;
+    const Level& lv = c->lv;
+    for (int d = 0; d < lv.dim; d += 2) {
+        Timed tm(c, names[mixed][d]);
+        launch_pass_solid<R, false>(c, in, d, F);
+    }
+    using T = STile<2, R>;
+    const unsigned g = grid1(lv.n[0], T::TC) * grid1(lv.n[1], T::PER - 1) * (unsigned)lv.n[2];
+    Timed tm(c, names[mixed][1]);
+    if (lv.dim == 2)
+        hipLaunchKernelGGL((k_stage1_s<2, 2, false, R>), dim3(g), dim3(256), 0, c->stream, lv, in, out, F[0], F[2], c->d_clk);
+    else
+        hipLaunchKernelGGL((k_stage1_s<2, 3, false, R>), dim3(g), dim3(256), 0, c->stream, lv, in, out, F[0], F[2], c->d_clk);
+}
 template <typename R, bool MX>
 static void launch_pass_t(tj_ctx* c, const MF& Uin, int d, const FacesT<R>* F, const Hist& h) {
     const Level& lv = c->lv;
@@ -1006,6 +1026,17 @@ static int launch_stage1d(tj_ctx* c, int stage, const MF& in, const MF& base, co
     return TJ_OK;
 }
 
+// Solid levels of two or three dimensions without Romenskii or Wilkins
+// materials: stage 1 with the y pass and the update in one launch, its output
+// in another buffer than its input (the kernel reads rows around each tile).
+static bool use_stage1_solid(const tj_ctx* c) { return c->stage2d && c->lv.solid && c->lv.dim >= 2 && !rw_level(c->lv); }
+static int launch_stage1_solid(tj_ctx* c, const MF& in, const MF& out, int prec) {
+    if (prec == TJ_PREC_MIXED) launch_stage1_solid_t<float>(c, in, out, c->Ff);
+    else launch_stage1_solid_t<double>(c, in, out, c->F);
+    HIPCHK(c, hipGetLastError());
+    return TJ_OK;
+}
+
 int tj_rk_stage(tj_ctx* c, int stage, const tj_mf* Uin, const tj_mf* Ubase, tj_mf* Uout, int prec) {
     if (!c || !c->bound) return TJ_ENOLEVEL;
     TJ_FORWARD_FABS(c, tj_rk_stage(c, stage, Uin, Ubase, Uout, prec), Uin, Ubase, Uout);
@@ -1019,6 +1050,7 @@ int tj_rk_stage(tj_ctx* c, int stage, const tj_mf* Uin, const tj_mf* Ubase, tj_m
     // the y kernel reads rows of Uin around each tile while other tiles write
     // Uout: an in-place stage (Uout == Uin) takes the flux-plane passes
     if (use_stage2d(c) && !same_view(view(Uout), in)) return launch_stage2d(c, stage, in, base, view(Uout), 0u, prec);
+    if (stage == 1 && use_stage1_solid(c) && !same_view(view(Uout), in)) return launch_stage1_solid(c, in, view(Uout), prec);
     if (use_stage1d(c) && !same_view(view(Uout), in)) return launch_stage1d(c, stage, in, base, view(Uout), 0u, false, prec);
     const FuseArgs fz{stage, base, view(Uout), 0u};
     bool fused = false;
@@ -1093,10 +1125,14 @@ int tj_step(tj_ctx* c, tj_mf* S, tj_mf* T, int prec) {
     }
     bool fused = false;
     const FuseArgs f1{1, s, t, 0u};
-    if ((r = launch_fluxes(c, s, &f1, &fused, prec))) return r;
-    if (!fused) {
-        Timed tm(c, mixed ? "update_stage1_mixed" : "update_stage1");
-        launch_update(c, 1, s, s, t, 0u, prec);
+    if (use_stage1_solid(c)) {
+        if ((r = launch_stage1_solid(c, s, t, prec))) return r;
+    } else {
+        if ((r = launch_fluxes(c, s, &f1, &fused, prec))) return r;
+        if (!fused) {
+            Timed tm(c, mixed ? "update_stage1_mixed" : "update_stage1");
+            launch_update(c, 1, s, s, t, 0u, prec);
+        }
     }
     const FuseArgs f2{2, s, s, step_ops(c)};
     if ((r = launch_fluxes(c, t, &f2, &fused, prec))) return r;
@@ -1657,7 +1693,7 @@ size_t carve_level(tj_ctx* c, const tj_level_desc* d, unsigned char* base, int p
         c->d_edge[a] = cv.take<uint8_t>(lv.n[a]);
         lv.edge[a] = c->d_edge[a];
     }
-    c->nfc = d->SOLID ? 3 * d->nmat + 17 : 2 * d->nmat + 5 + (lv.mixm >= 0 ? 1 : 0);
+    c->nfc = d->SOLID ? 3 * d->nmat + 14 : 2 * d->nmat + 5 + (lv.mixm >= 0 ? 1 : 0);
     for (int a = 0; a < d->dim; ++a) {
         Faces& F = c->F[a];
         F.nx = lv.n[0] + (a == 0);

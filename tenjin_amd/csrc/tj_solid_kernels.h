@@ -59,6 +59,37 @@ __device__ __forceinline__ SSt<NM, R> state_dn(const SSt<NM, R>& S) {
 template <int NM, typename R>
 __device__ __forceinline__ void flip_s(SSt<NM, R>& S, int d) { S.u[d] = -S.u[d]; }
 
+// The flux planes of direction D hold what the update reads of wave5's flux:
+// alpha, alpha rho, rho u, E, the two rows of V other than D (row D's flux is
+// V_D u_D - V_D u_D = 0 and its jumps are 0), alpha rho epsilon, S* and row D
+// of V*.  20 of 23 components: 72 of the 984 and 1208 bytes a cell that the
+// FP64 update stages moved at the device's copy rate.
+template <int NM>
+struct SFace {
+    static constexpr int N = 3 * NM + 14;
+    static constexpr int ARE = 2 * NM + 10, SS = 3 * NM + 10, VS = 3 * NM + 11;
+    // component of V row r (r != d), column c
+    static constexpr int v(int d, int r, int c) { return 2 * NM + 4 + 3 * (r > d ? r - 1 : r) + c; }
+};
+// put(q, x) for each plane q of direction D, from wave5's flux
+template <int NM, int D, typename R, typename Put>
+__device__ __forceinline__ void put_face(const R* Fv, Put put) {
+    using S = SFace<NM>;
+    constexpr int NC = 3 * NM + 13;
+#pragma unroll
+    for (int q = 0; q < 2 * NM + 4; ++q) put(q, Fv[q]);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            if (r != D) put(S::v(D, r, c), Fv[2 * NM + 4 + r * 3 + c]);
+#pragma unroll
+    for (int m = 0; m < NM; ++m) put(S::ARE + m, Fv[2 * NM + 13 + m]);
+    put(S::SS, Fv[NC]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) put(S::VS + c, Fv[NC + 1 + c]);
+}
+
 // Flux passes of the solid path, one reconstruction per cell: a lane
 // reconstructs one cell (MUSCL, then p2c + sound speed of both face states)
 // and face f takes its left state UR(f-1) from lane - 1, the cell one below
@@ -103,7 +134,6 @@ template <int NM, int LN, bool RW, typename R>
 __global__ __launch_bounds__(256) void k_flux_x_s(Level lv, MF U, FacesT<R> F, Clock* clk) {
     if (clk->done) return;
     constexpr int PER = LN - 1;
-    constexpr int NF = 3 * NM + 17;
     const int lane = threadIdx.x & 63, ld = lane % LN;
     const long long wave = xcd_block(blockIdx.x, gridDim.x, 2) * (blockDim.x >> 6) + wave_in_block();
     const int nx = lv.n[0], ny = lv.n[1];
@@ -127,12 +157,12 @@ __global__ __launch_bounds__(256) void k_flux_x_s(Level lv, MF U, FacesT<R> F, C
         muscl_s<NM, R>(Pm, Pc, Pp, PL, PR);
     }
     unsigned st = 0;
-    R Fv[NF];
+    R Fv[3 * NM + 17];
     const bool face = act && ld >= 1 && c >= 0 && c <= nx;
     face_s<NM, 0, RW, R>(lv, PL, PR, c, face, Fv, st);
     if (face) {
-#pragma unroll
-        for (int q = 0; q < NF; ++q) F.at(q, c, j, k) = Fv[q];
+        const long long id = ((long long)k * F.ny + j) * F.nx + c;
+        put_face<NM, 0>(Fv, [&](int q, R x) { F.p[q * F.cs + id] = x; });
     }
     if (st) atomicOr(&clk->status, st);
 }
@@ -150,23 +180,18 @@ struct STile {
     static constexpr int PER = LN - 1;           // faces per segment
     static constexpr int ROWS = LN + 2;          // rows c0 - 1 .. c0 + LN
     static constexpr int NP = 3 * NM + 13;       // primitives
-    static constexpr int NF = 3 * NM + 17;       // flux components
+    static constexpr int NF = SFace<NM>::N;      // flux planes
     static constexpr int FR = PER + 2;           // column pitch of the staged fluxes
     static constexpr int WORDS = NP * TC * ROWS > NF * TC * FR ? NP * TC * ROWS : NF * TC * FR;
 };
+// The fluxes of faces c0 + 1 .. c0 + 15 along D of columns i0 .. i0 + 15, o the
+// other index: left in lds, plane q of column col and face c0 + 1 + f at
+// (q * TC + col) * FR + f, with a barrier at the end.
 template <int NM, int D, bool RW, typename R>
-__global__ __launch_bounds__(256) void k_flux_yz_s(Level lv, MF U, FacesT<R> F, Clock* clk) {
+__device__ __forceinline__ void tile_faces_s(const Level& lv, const MF& U, R* lds, int i0, int c0, int o, unsigned& st) {
     using T = STile<NM, R>;
-    constexpr int TC = T::TC, LN = T::LN, PER = T::PER, ROWS = T::ROWS, NF = T::NF, FR = T::FR;
-    __shared__ R lds[T::WORDS];
-    if (clk->done) return;  // uniform: the clock does not change during the launch
-    const int nx = lv.n[0], ny = lv.n[1], nd = lv.n[D];
-    const int nxt = (nx + TC - 1) / TC, nseg = (nd + 1 + PER - 1) / PER;
-    const long long tile = xcd_block(blockIdx.x, gridDim.x, 2);
-    const int xt = (int)(tile % nxt);
-    const int rest = (int)(tile / nxt);
-    const int seg = rest % nseg, o = rest / nseg;
-    const int i0 = xt * TC, c0 = seg * PER - 1;
+    constexpr int TC = T::TC, LN = T::LN, ROWS = T::ROWS, FR = T::FR;
+    const int nx = lv.n[0], nd = lv.n[D];
     const int tid = threadIdx.x;
     auto P = [&](int q, int col, int t) -> R& { return lds[(q * TC + col) * ROWS + t]; };
     // one cell of the first 16 rows per thread; then the two rows left, their
@@ -242,25 +267,36 @@ __global__ __launch_bounds__(256) void k_flux_yz_s(Level lv, MF U, FacesT<R> F, 
         get(t + 1, Pp);
         muscl_s<NM, R>(Pm, Pc, Pp, PL, PR);
     }
-    unsigned st = 0;
-    R Fv[NF];
+    R Fv[3 * NM + 17];
     const bool face = i0 + col < nx && ld >= 1 && c >= 0 && c <= nd;
     face_s<NM, D, RW, R>(lv, PL, PR, c, face, Fv, st);
     __syncthreads();  // every wave has read its primitives: the fluxes may overwrite them
-    if (face) {
-#pragma unroll
-        for (int q = 0; q < NF; ++q) lds[(q * TC + col) * FR + ld - 1] = Fv[q];
-    }
+    if (face) put_face<NM, D>(Fv, [&](int q, R x) { lds[(q * TC + col) * FR + ld - 1] = x; });
     __syncthreads();
-    {
-        const int cc = tid % TC, f = tid / TC;  // column, face of the segment
-        const int ii = i0 + cc, cf = c0 + 1 + f;
-        if (f < PER && ii < nx && cf <= nd) {
-            const int fj = D == 1 ? cf : o, fk = D == 2 ? cf : o;
-            const long long id = ((long long)fk * F.ny + fj) * F.nx + ii;
+}
+template <int NM, int D, bool RW, typename R>
+__global__ __launch_bounds__(256) void k_flux_yz_s(Level lv, MF U, FacesT<R> F, Clock* clk) {
+    using T = STile<NM, R>;
+    constexpr int TC = T::TC, PER = T::PER, NF = T::NF, FR = T::FR;
+    __shared__ R lds[T::WORDS];
+    if (clk->done) return;  // uniform: the clock does not change during the launch
+    const int nx = lv.n[0], nd = lv.n[D];
+    const int nxt = (nx + TC - 1) / TC, nseg = (nd + 1 + PER - 1) / PER;
+    const long long tile = xcd_block(blockIdx.x, gridDim.x, 2);
+    const int xt = (int)(tile % nxt);
+    const int rest = (int)(tile / nxt);
+    const int seg = rest % nseg, o = rest / nseg;
+    const int i0 = xt * TC, c0 = seg * PER - 1;
+    const int tid = threadIdx.x;
+    unsigned st = 0;
+    tile_faces_s<NM, D, RW, R>(lv, U, lds, i0, c0, o, st);
+    const int cc = tid % TC, f = tid / TC;  // column, face of the segment
+    const int ii = i0 + cc, cf = c0 + 1 + f;
+    if (f < PER && ii < nx && cf <= nd) {
+        const int fj = D == 1 ? cf : o, fk = D == 2 ? cf : o;
+        const long long id = ((long long)fk * F.ny + fj) * F.nx + ii;
 #pragma unroll
-            for (int q = 0; q < NF; ++q) F.p[q * F.cs + id] = lds[(q * TC + cc) * FR + f];
-        }
+        for (int q = 0; q < NF; ++q) F.p[q * F.cs + id] = lds[(q * TC + cc) * FR + f];
     }
     if (st) atomicOr(&clk->status, st);
 }
@@ -358,16 +394,128 @@ __device__ __forceinline__ void radial_solid_c2p(const Level& lv, double f, SCel
     C.hj2 = c2p_s<NM, RW>(lv, C.al, C.ar, C.are, C.ru, C.E, C.V, C.rk, C.e, C.rho, C.u, C.p, dH);
 }
 
-// update (hllc.cpp:493-523, with the V rows of :511-514) in x, y, z order,
+// update_cell_s: update (hllc.cpp:493-523, with the V rows of :511-514) in x, y, z order,
 // then conservativeToPrimitive.  Stage 2 adds the RK average (hllc.cpp:705),
 // plasticUpdate (main.cpp:154-157, plastic.cpp:227-244), the geometric source
 // (main.cpp:159-162), cleanUpV (main.cpp:164-167), cleanUpAlpha
 // (main.cpp:169-171), the NaN scan and the next getTimeStep.
+// fa(d, q, hi): plane q of the cell's low (0) or high (1) face along d < ND.
+template <int NM, int STAGE, bool RW, typename T, int ND = 3, typename Face>
+__device__ __forceinline__ void update_cell_s(const Level& lv, const MF& Uin, const MF& Ub, const MF& Uo, int i, int j,
+                                              int k, double dt, unsigned ops, Face fa, double& cand, unsigned& st) {
+    using S = SFace<NM>;
+    SCell<NM> C;
+    load_scell<NM, true>(lv, Uin, i, j, k, C);
+    double a0[NM], V0[9], u0[3];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) a0[m] = C.al[m];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) V0[q] = C.V[q];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) u0[q] = C.u[q];
+    // unrolled over the directions (a loop to lv.dim kept C.are in scratch
+    // memory: the plastic-only update made its index dynamic)
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        if (d >= lv.dim) break;
+        const double dtdx = dt / lv.dx[d];
+        const double s0 = (double)fa(d, S::SS, 0), s1 = (double)fa(d, S::SS, 1);
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            C.al[m] += dtdx * ((double)fa(d, m, 0) - (double)fa(d, m, 1) - a0[m] * (s0 - s1));
+            C.ar[m] += dtdx * ((double)fa(d, NM + m, 0) - (double)fa(d, NM + m, 1));
+            if (lv.plastic) {
+                const double fl = (double)fa(d, S::ARE + m, 0), fh = (double)fa(d, S::ARE + m, 1);
+                C.are[m] += dtdx * (fl - fh);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) C.ru[q] += dtdx * ((double)fa(d, 2 * NM + q, 0) - (double)fa(d, 2 * NM + q, 1));
+        C.E += dtdx * ((double)fa(d, 2 * NM + 3, 0) - (double)fa(d, 2 * NM + 3, 1));
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const double vs0 = (double)fa(d, S::VS + c, 0), vs1 = (double)fa(d, S::VS + c, 1);
+                const double jump = r == d ? 0.0 : (double)fa(d, S::v(d, r, c), 0) - (double)fa(d, S::v(d, r, c), 1);
+                C.V[r * 3 + c] += dtdx * (jump - (2.0 / 3.0) * V0[r * 3 + c] * (s0 - s1) + u0[r] * (vs0 - vs1));
+            }
+    }
+    double dH[9];
+    // Stage 2 with the plastic relaxation: the conservativeToPrimitive that
+    // ends it rewrites rho, u, p, HJ2 and dH, so this one forms only what
+    // the relaxation reads (rho_k and epsilon, as c2p_s does).  The values
+    // are those of the full sequence.
+    const bool relax = STAGE == 2 && (ops & 1u) != 0;
+    SCell<NM> B;
+    if (STAGE == 2) load_scell<NM, true>(lv, Ub, i, j, k, B);  // in flight across the branch
+    if (relax) {  // nor are these averages read (156 VGPRs, three waves per SIMD; 171 with them)
+        B.rho = B.p = B.hj2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) B.u[q] = 0.0;
+    }
+    if (relax) {
+        c2p_rk_e<NM>(lv, C.al, C.ar, C.are, C.rk, C.e);
+        C.rho = C.p = C.hj2 = 0.0;  // rewritten after the relaxation (no loads of Uin's values)
+    } else C.hj2 = c2p_s<NM, RW>(lv, C.al, C.ar, C.are, C.ru, C.E, C.V, C.rk, C.e, C.rho, C.u, C.p, dH);
+    if (STAGE == 2) {
+        // U1 = (U * 1/2) + (U2 * 1/2) over every component
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            C.al[m] = B.al[m] * (1.0 / 2.0) + C.al[m] * (1.0 / 2.0);
+            C.ar[m] = B.ar[m] * (1.0 / 2.0) + C.ar[m] * (1.0 / 2.0);
+            C.rk[m] = B.rk[m] * (1.0 / 2.0) + C.rk[m] * (1.0 / 2.0);
+            C.e[m] = B.e[m] * (1.0 / 2.0) + C.e[m] * (1.0 / 2.0);
+            C.are[m] = B.are[m] * (1.0 / 2.0) + C.are[m] * (1.0 / 2.0);
+        }
+        C.rho = B.rho * (1.0 / 2.0) + C.rho * (1.0 / 2.0);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            C.ru[q] = B.ru[q] * (1.0 / 2.0) + C.ru[q] * (1.0 / 2.0);
+            C.u[q] = B.u[q] * (1.0 / 2.0) + C.u[q] * (1.0 / 2.0);
+        }
+        C.E = B.E * (1.0 / 2.0) + C.E * (1.0 / 2.0);
+        C.p = B.p * (1.0 / 2.0) + C.p * (1.0 / 2.0);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) C.V[q] = B.V[q] * (1.0 / 2.0) + C.V[q] * (1.0 / 2.0);
+        C.hj2 = B.hj2 * (1.0 / 2.0) + C.hj2 * (1.0 / 2.0);
+        if (relax) {  // plastic relaxation, then conservativeToPrimitive
+            st |= plastic_cell<NM, RW>(lv, C.al, C.ar, C.rk, C.e, C.are, C.V);
+            C.hj2 = c2p_s<NM, RW>(lv, C.al, C.ar, C.are, C.ru, C.E, C.V, C.rk, C.e, C.rho, C.u, C.p, dH);
+        }
+        if (ops & 32u) radial_solid_c2p<NM, RW>(lv, radial_factor(lv, i, dt), C, dH, (ops & 1u) != 0);
+        if (ops & 2u) cleanup_v<NM, T>(lv, C.al, C.V);  // FP32 in the mixed form
+        if (ops & 4u) st |= cleanup_alpha<NM>(C.al);
+        if (ops & 16u) {
+            bool bad = false;
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+                bad |= __builtin_isnan(C.al[m]) || __builtin_isnan(C.ar[m]) || __builtin_isnan(C.rk[m]) ||
+                       (lv.plastic && (__builtin_isnan(C.e[m]) || __builtin_isnan(C.are[m])));
+#pragma unroll
+            for (int q = 0; q < 3; ++q) bad |= __builtin_isnan(C.ru[q]) || __builtin_isnan(C.u[q]);
+#pragma unroll
+            for (int q = 0; q < 9; ++q) bad |= __builtin_isnan(C.V[q]);
+            bad |= __builtin_isnan(C.E) || __builtin_isnan(C.p);
+            if (bad) st |= 1u;
+        }
+        if (ops & 8u) {
+            const double a = sound_s<NM, RW>(lv, C.al, C.ar, C.rk, C.rho, C.p, C.hj2);
+            put_state<STAGE == 2>(Uo.at(lv.cs[SOUNDSPEED], i, j, k), a);
+            #pragma unroll
+            for (int d = 0; d < 3; ++d)  // unrolled: constant indices keep the state in registers
+                if (d < lv.dim) cand = dmin(cand, qdiv(lv.dx[d], a + __builtin_fabs(C.u[d])));
+        }
+    }
+    store_scell<NM, STAGE == 2>(lv, Uo, i, j, k, C);
+}
+
+// Bound by HBM: with 20 flux planes a direction in place of 23, stage 1 of
+// 144^3 FP64 takes 575 us (605), stage 2 715 (760).
 template <int NM, int STAGE, bool RW, typename T>
 __global__ __launch_bounds__(256) void k_update_s(Level lv, MF Uin, MF Ub, MF Uo, FacesT<T> F0, FacesT<T> F1, FacesT<T> F2,
                                                   Clock* clk, unsigned ops) {
     if (clk->done) return;
-    constexpr int NC = 3 * NM + 13;
     const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
     const long long id = xcd_block(blockIdx.x, gridDim.x, lv.dim) * blockDim.x + threadIdx.x;
     const long long ncell = (long long)nx * ny * nz;
@@ -377,112 +525,51 @@ __global__ __launch_bounds__(256) void k_update_s(Level lv, MF Uin, MF Ub, MF Uo
         const int i = (int)(id % nx);
         const int j = (int)((id / nx) % ny);
         const int k = (int)(id / ((long long)nx * ny));
-        const double dt = clk->dt;
-        SCell<NM> C;
-        load_scell<NM, true>(lv, Uin, i, j, k, C);
-        double a0[NM], V0[9], u0[3];
-#pragma unroll
-        for (int m = 0; m < NM; ++m) a0[m] = C.al[m];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) V0[q] = C.V[q];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) u0[q] = C.u[q];
-        // unrolled over the three directions (a loop to lv.dim kept C.are in
-        // scratch memory: the plastic-only update made its index dynamic)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            if (d >= lv.dim) break;
-            const FacesT<T>& Fd = d == 0 ? F0 : (d == 1 ? F1 : F2);
-            const int i1 = i + (d == 0), j1 = j + (d == 1), k1 = k + (d == 2);
-            const double dtdx = dt / lv.dx[d];
-            const double s0 = (double)Fd.at(NC, i, j, k), s1 = (double)Fd.at(NC, i1, j1, k1);
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                C.al[m] += dtdx * ((double)Fd.at(m, i, j, k) - (double)Fd.at(m, i1, j1, k1) - a0[m] * (s0 - s1));
-                C.ar[m] += dtdx * ((double)Fd.at(NM + m, i, j, k) - (double)Fd.at(NM + m, i1, j1, k1));
-                if (lv.plastic) {
-                    const double fl = (double)Fd.at(2 * NM + 13 + m, i, j, k), fh = (double)Fd.at(2 * NM + 13 + m, i1, j1, k1);
-                    C.are[m] += dtdx * (fl - fh);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 3; ++q) C.ru[q] += dtdx * ((double)Fd.at(2 * NM + q, i, j, k) - (double)Fd.at(2 * NM + q, i1, j1, k1));
-            C.E += dtdx * ((double)Fd.at(2 * NM + 3, i, j, k) - (double)Fd.at(2 * NM + 3, i1, j1, k1));
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const int n = 2 * NM + 4 + r * 3 + c;
-                    const double vs0 = (double)Fd.at(NC + 1 + c, i, j, k), vs1 = (double)Fd.at(NC + 1 + c, i1, j1, k1);
-                    C.V[r * 3 + c] += dtdx * ((double)Fd.at(n, i, j, k) - (double)Fd.at(n, i1, j1, k1) - (2.0 / 3.0) * V0[r * 3 + c] * (s0 - s1) +
-                                              u0[r] * (vs0 - vs1));
-                }
-        }
-        double dH[9];
-        // Stage 2 with the plastic relaxation: the conservativeToPrimitive that
-        // ends it rewrites rho, u, p, HJ2 and dH, so this one forms only what
-        // the relaxation reads (rho_k and epsilon, as c2p_s does).  The values
-        // are those of the full sequence.
-        const bool relax = STAGE == 2 && (ops & 1u) != 0;
-        SCell<NM> B;
-        if (STAGE == 2) load_scell<NM, true>(lv, Ub, i, j, k, B);  // in flight across the branch
-        if (relax) {
-            c2p_rk_e<NM>(lv, C.al, C.ar, C.are, C.rk, C.e);
-            C.rho = C.p = C.hj2 = 0.0;  // rewritten after the relaxation (no loads of Uin's values)
-        } else C.hj2 = c2p_s<NM, RW>(lv, C.al, C.ar, C.are, C.ru, C.E, C.V, C.rk, C.e, C.rho, C.u, C.p, dH);
-        if (STAGE == 2) {
-            // U1 = (U * 1/2) + (U2 * 1/2) over every component
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                C.al[m] = B.al[m] * (1.0 / 2.0) + C.al[m] * (1.0 / 2.0);
-                C.ar[m] = B.ar[m] * (1.0 / 2.0) + C.ar[m] * (1.0 / 2.0);
-                C.rk[m] = B.rk[m] * (1.0 / 2.0) + C.rk[m] * (1.0 / 2.0);
-                C.e[m] = B.e[m] * (1.0 / 2.0) + C.e[m] * (1.0 / 2.0);
-                C.are[m] = B.are[m] * (1.0 / 2.0) + C.are[m] * (1.0 / 2.0);
-            }
-            C.rho = B.rho * (1.0 / 2.0) + C.rho * (1.0 / 2.0);
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                C.ru[q] = B.ru[q] * (1.0 / 2.0) + C.ru[q] * (1.0 / 2.0);
-                C.u[q] = B.u[q] * (1.0 / 2.0) + C.u[q] * (1.0 / 2.0);
-            }
-            C.E = B.E * (1.0 / 2.0) + C.E * (1.0 / 2.0);
-            C.p = B.p * (1.0 / 2.0) + C.p * (1.0 / 2.0);
-#pragma unroll
-            for (int q = 0; q < 9; ++q) C.V[q] = B.V[q] * (1.0 / 2.0) + C.V[q] * (1.0 / 2.0);
-            C.hj2 = B.hj2 * (1.0 / 2.0) + C.hj2 * (1.0 / 2.0);
-            if (relax) {  // plastic relaxation, then conservativeToPrimitive
-                st |= plastic_cell<NM, RW>(lv, C.al, C.ar, C.rk, C.e, C.are, C.V);
-                C.hj2 = c2p_s<NM, RW>(lv, C.al, C.ar, C.are, C.ru, C.E, C.V, C.rk, C.e, C.rho, C.u, C.p, dH);
-            }
-            if (ops & 32u) radial_solid_c2p<NM, RW>(lv, radial_factor(lv, i, dt), C, dH, (ops & 1u) != 0);
-            if (ops & 2u) cleanup_v<NM, T>(lv, C.al, C.V);  // FP32 in the mixed form
-            if (ops & 4u) st |= cleanup_alpha<NM>(C.al);
-            if (ops & 16u) {
-                bool bad = false;
-#pragma unroll
-                for (int m = 0; m < NM; ++m)
-                    bad |= __builtin_isnan(C.al[m]) || __builtin_isnan(C.ar[m]) || __builtin_isnan(C.rk[m]) ||
-                           (lv.plastic && (__builtin_isnan(C.e[m]) || __builtin_isnan(C.are[m])));
-#pragma unroll
-                for (int q = 0; q < 3; ++q) bad |= __builtin_isnan(C.ru[q]) || __builtin_isnan(C.u[q]);
-#pragma unroll
-                for (int q = 0; q < 9; ++q) bad |= __builtin_isnan(C.V[q]);
-                bad |= __builtin_isnan(C.E) || __builtin_isnan(C.p);
-                if (bad) st |= 1u;
-            }
-            if (ops & 8u) {
-                const double a = sound_s<NM, RW>(lv, C.al, C.ar, C.rk, C.rho, C.p, C.hj2);
-                put_state<STAGE == 2>(Uo.at(lv.cs[SOUNDSPEED], i, j, k), a);
-                #pragma unroll
-                for (int d = 0; d < 3; ++d)  // unrolled: constant indices keep the state in registers
-                    if (d < lv.dim) cand = dmin(cand, qdiv(lv.dx[d], a + __builtin_fabs(C.u[d])));
-            }
-        }
-        store_scell<NM, STAGE == 2>(lv, Uo, i, j, k, C);
+        update_cell_s<NM, STAGE, RW, T>(lv, Uin, Ub, Uo, i, j, k, clk->dt, ops, [&](int d, int q, int hi) {
+            const FacesT<T>& F = d == 0 ? F0 : (d == 1 ? F1 : F2);
+            return F.at(q, i + (d == 0 && hi), j + (d == 1 && hi), k + (d == 2 && hi));
+        }, cand, st);
     }
     if (STAGE == 2 && (ops & 8u)) {
         block_min_to(cand, dt_slot(lv, clk));
+    }
+    if (st) atomicOr(&clk->status, st);
+}
+
+// The y flux pass and the update of stage 1 in one launch: the tile's y faces
+// stay in LDS and the update takes the other directions' faces from their
+// planes.  A tile gives 15 faces and completes the 14 cells between them, lanes
+// along x again.  The update alone is bound by HBM and the pass by VALU issue:
+// 144^3 FP64 430 + 575 us as two launches, 790 as one; 512^2 50 + 31 and 69.
+// Stage 2 stays apart: its update has as much arithmetic as a pass and takes
+// three waves per SIMD alone, two here (144^3 FP64 1363 against 1135 us, FP32
+// fluxes on 203 x 160 x 131 1640 against 1010).  With the z pass in the place
+// of y, whose tile rows lie whole planes apart, stage 1 takes 800 and 890 us
+// against 781 and 826.  DIM: the level's dimensions.
+template <int NM, int DIM, bool RW, typename R>
+__global__ __launch_bounds__(256) void k_stage1_s(Level lv, MF U, MF Uo, FacesT<R> F0, FacesT<R> F2, Clock* clk) {
+    using T = STile<NM, R>;
+    constexpr int TC = T::TC, FR = T::FR, PER = T::PER - 1;
+    __shared__ R lds[T::WORDS];
+    if (clk->done) return;  // uniform: the clock does not change during the launch
+    const int nx = lv.n[0], ny = lv.n[1];
+    const int nxt = (nx + TC - 1) / TC, nseg = (ny + PER - 1) / PER;
+    const long long tile = xcd_block(blockIdx.x, gridDim.x, 2);
+    const int xt = (int)(tile % nxt);
+    const int rest = (int)(tile / nxt);
+    const int seg = rest % nseg, k = rest / nseg;
+    const int i0 = xt * TC, c0 = seg * PER - 1;
+    const int tid = threadIdx.x;
+    double cand = __builtin_huge_val();
+    unsigned st = 0;
+    tile_faces_s<NM, 1, RW, R>(lv, U, lds, i0, c0, k, st);
+    const int cc = tid % TC, f = tid / TC;
+    const int i = i0 + cc, j = c0 + 1 + f;
+    if (f < PER && i < nx && j < ny) {
+        update_cell_s<NM, 1, RW, R, DIM>(lv, U, U, Uo, i, j, k, clk->dt, 0u, [&](int d, int q, int hi) {
+            if (d == 1) return lds[(q * TC + cc) * FR + f + hi];
+            return d == 0 ? F0.at(q, i + hi, j, k) : F2.at(q, i, j, k + hi);
+        }, cand, st);
     }
     if (st) atomicOr(&clk->status, st);
 }
