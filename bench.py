@@ -53,10 +53,12 @@ FLUID_KERNEL_BYTES = {
     "xstage2": 112 + 64 + 16,
     "ystage1": 64 + 64 + 16 + 120,
     "ystage2_post": 64 + 64 + 16 + 120 + 120 + 8,
-    "xstage1_mixed": 112 + 64 + 16,
-    "xstage2_mixed": 112 + 64 + 16,
-    "ystage1_mixed": 64 + 64 + 16 + 120,
-    "ystage2_post_mixed": 64 + 64 + 16 + 120 + 120 + 8,
+    # mixed form: FP32 x faces (9 comps) in place of the partial state, the
+    # further conserved comps read by the y kernel
+    "xstage1_mixed": 64 + 36 + 16,
+    "xstage2_mixed": 64 + 36 + 16,
+    "ystage1_mixed": 112 + 36 + 16 + 120,
+    "ystage2_post_mixed": 112 + 36 + 16 + 120 + 120 + 8,
     "flux_x": 64 + 72 + 16,            # 8 primitives in, 9 flux comps out, 2 star alphas out
     "flux_y": 64 + 72 + 16,
     "flux_z": 64 + 72,
@@ -83,10 +85,10 @@ MIX_KERNEL_BYTES = {
     "xstage2": 128 + 72 + 16,
     "ystage1": 72 + 72 + 16 + 152,
     "ystage2_post": 72 + 72 + 16 + 152 + 152 + 8,
-    "xstage1_mixed": 128 + 72 + 16,
-    "xstage2_mixed": 128 + 72 + 16,
-    "ystage1_mixed": 72 + 72 + 16 + 152,
-    "ystage2_post_mixed": 72 + 72 + 16 + 152 + 152 + 8,
+    "xstage1_mixed": 72 + 40 + 16,
+    "xstage2_mixed": 72 + 40 + 16,
+    "ystage1_mixed": 128 + 40 + 16 + 152,
+    "ystage2_post_mixed": 128 + 40 + 16 + 152 + 152 + 8,
     "flux_x": 72 + 80 + 16,
     "flux_y": 72 + 80 + 16,
     "update_stage1": 72 + 2 * 80 + 152,

@@ -92,7 +92,9 @@ __device__ __forceinline__ const FacesT<float>& bfaces<float>(const BProb& P, in
 // x pass over all problems of a group; which = 0 reads S, 1 reads T
 template <bool TH, typename R>
 __global__ __launch_bounds__(256) void k_b_flux_x(BTab t, int which, int q, int e) {
-    const long long gw = bwave();
+    // blocks renumbered per XCD as on a single 2D level (xcd_block): each
+    // XCD's L2 then holds neighbouring rows of one problem
+    const long long gw = xcd_block(blockIdx.x, gridDim.x, 2) * (blockDim.x >> 6) + wave_in_block();
     if (gw >= bunits(t)) return;
     const int p = bfind(t.start, t.np, gw);
     const BProb& P = ro_at(t.p, p);
@@ -135,20 +137,23 @@ __global__ __launch_bounds__(256) void k_b_update(BTab t, unsigned ops) {
     else update_body<2, 2, T>(P.lv, P.T, P.S, P.S, F0, F1, F0, P.clk, ops, gb - ro_at(t.start, p));
 }
 
-// stage kernels of the 2D problems (tj_stage2d.h): x part over all problems,
-// then the y part over the problems of one tile shape
-template <bool TH, typename R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && sizeof(R) == 8 ? 4 : 1)))
+// stage kernels of the 2D problems (tj_stage2d.h): x part over all problems
+// (mixed form: k_b_flux_x), then the y part over the problems of one tile shape
+template <bool TH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH ? 4 : 1)))
 void k_b_xstage(BTab t, int which, int q, int e) {
-    // blocks renumbered per XCD as on a single 2D level (xcd_block): each
-    // XCD's L2 then holds neighbouring rows of one problem
-    const long long gw = xcd_block(blockIdx.x, gridDim.x, 2) * (blockDim.x >> 6) +
-                         wave_in_block();
+    const long long gw = xcd_block(blockIdx.x, gridDim.x, 2) * (blockDim.x >> 6) + wave_in_block();
     if (gw >= bunits(t)) return;
     const int p = bfind(t.start, t.np, gw);
     const BProb& P = ro_at(t.p, p);
-    xstage_body<2, TH, R>(P.lv, which ? P.T : P.S, P.ux, bhist(P, 0, q, e), P.clk, gw - ro_at(t.start, p));
+    xstage_body<2, TH, double>(P.lv, which ? P.T : P.S, P.ux, bhist(P, 0, q, e), P.clk, gw - ro_at(t.start, p));
 }
+template <typename R>
+__device__ __forceinline__ const typename XPart<R>::T& bxpart(const BProb& P);
+template <>
+__device__ __forceinline__ const UxPlanes& bxpart<double>(const BProb& P) { return P.ux; }
+template <>
+__device__ __forceinline__ const FacesT<float>& bxpart<float>(const BProb& P) { return P.Ff[0]; }
 // one RK stage of every 1D problem in one launch (k_xstage1d of a single
 // level): reconstruction, fluxes and the completion of each wave's cells
 template <bool TH, int STAGE, typename R>
@@ -169,9 +174,9 @@ __global__ __launch_bounds__(TC * LPS) void k_b_ystage(BTab t, int q, int e, uns
     const int p = bfind(t.start, t.np, gb);
     const BProb& P = ro_at(t.p, p);
     if (STAGE == 1)
-        ystage_body<2, TH, TC, LPS, 1, R>(P.lv, P.S, P.ux, P.S, P.T, bhist(P, 1, q, e), P.clk, ops, gb - ro_at(t.start, p));
+        ystage_body<2, TH, TC, LPS, 1, R>(P.lv, P.S, bxpart<R>(P), P.S, P.T, bhist(P, 1, q, e), P.clk, ops, gb - ro_at(t.start, p));
     else
-        ystage_body<2, TH, TC, LPS, 2, R>(P.lv, P.T, P.ux, P.S, P.S, bhist(P, 1, q, e), P.clk, ops, gb - ro_at(t.start, p));
+        ystage_body<2, TH, TC, LPS, 2, R>(P.lv, P.T, bxpart<R>(P), P.S, P.S, bhist(P, 1, q, e), P.clk, ops, gb - ro_at(t.start, p));
 }
 
 __global__ __launch_bounds__(256) void k_b_sound_dt(BTab t) {
@@ -401,8 +406,12 @@ void launch_b_stage2d(tj_batch* b, int g, int stage, unsigned ops) {
     const int which = stage == 1 ? 0 : 1;
     {
         const int q = (int)(b->pass[g] & 1), e = (int)(b->dpass[g][0] & 1);
-        hipLaunchKernelGGL((k_b_xstage<TH, R>), dim3(grid1(b->tot[g][3], 4)), dim3(256), 0, b->stream, tab(b, g, 3), which,
-                           q, e);
+        if constexpr (sizeof(R) == 4)
+            hipLaunchKernelGGL((k_b_flux_x<TH, R>), dim3(grid1(b->tot[g][0], 4)), dim3(256), 0, b->stream, tab(b, g, 0),
+                               which, q, e);
+        else
+            hipLaunchKernelGGL((k_b_xstage<TH>), dim3(grid1(b->tot[g][3], 4)), dim3(256), 0, b->stream, tab(b, g, 3),
+                               which, q, e);
         if (b->thinc) {
             b->pass[g] += 1;
             b->dpass[g][0] += 1;

@@ -32,6 +32,22 @@ __device__ __forceinline__ unsigned long long* dt_slot(const Level& lv, Clock* c
 // Everything below takes or launches with the state view MF (see tj_device.h).
 inline namespace TJ_VIEW_NS {
 
+// ------------------------------------------------------------------ XCD-aware block order
+// The 8 XCDs of the device take a grid's blocks round-robin (block b runs on
+// XCD b mod 8) and each XCD has its own L2.  Renumbering blocks so that each
+// XCD works through one contiguous range of cells keeps a 2D level's
+// neighbouring rows, which share their faces, in one L2 (measured: the 2D
+// update kernels 6-8 % faster).  In 3D the round-robin order is kept: with
+// 256 cells per row the cell above in z is 256 blocks on, which round-robin
+// puts on the same XCD one generation of resident blocks later, while the
+// contiguous order would put it out of the L2 (measured slower).
+__device__ __forceinline__ long long xcd_block(long long b, long long nb, int dim) {
+    if (dim > 2) return b;
+    const long long base = nb / 8, extra = nb % 8;
+    const long long x = b % 8, q = b / 8;
+    return x * base + (x < extra ? x : extra) + q;  // a bijection of [0, nb)
+}
+
 // ------------------------------------------------------------------ x pass
 // One wave covers a row segment; lane l holds cell c = f0 - H + l.  Lanes
 // reconstruct their cell (at the boundary-mapped cell s), neighbours' data
@@ -169,23 +185,8 @@ __device__ __forceinline__ void flux_x_body(const Level& lv, const MF& U, const 
 template <int NM, bool TH, typename R = double, bool MX = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && !MX && sizeof(R) == 8 ? 4 : 1)))
 void k_flux_x(Level lv, MF U, FacesT<R> F, Hist h, Clock* clk) {
-    flux_x_body<NM, TH, R, MX>(lv, U, F, h, clk, (long long)blockIdx.x * (blockDim.x >> 6) + wave_in_block());
-}
-
-// ------------------------------------------------------------------ XCD-aware block order
-// The 8 XCDs of the device take a grid's blocks round-robin (block b runs on
-// XCD b mod 8) and each XCD has its own L2.  Renumbering blocks so that each
-// XCD works through one contiguous range of cells keeps a 2D level's
-// neighbouring rows, which share their faces, in one L2 (measured: the 2D
-// update kernels 6-8 % faster).  In 3D the round-robin order is kept: with
-// 256 cells per row the cell above in z is 256 blocks on, which round-robin
-// puts on the same XCD one generation of resident blocks later, while the
-// contiguous order would put it out of the L2 (measured slower).
-__device__ __forceinline__ long long xcd_block(long long b, long long nb, int dim) {
-    if (dim > 2) return b;
-    const long long base = nb / 8, extra = nb % 8;
-    const long long x = b % 8, q = b / 8;
-    return x * base + (x < extra ? x : extra) + q;  // a bijection of [0, nb)
+    const long long b = xcd_block(blockIdx.x, gridDim.x, lv.dim);
+    flux_x_body<NM, TH, R, MX>(lv, U, F, h, clk, b * (blockDim.x >> 6) + wave_in_block());
 }
 
 // ------------------------------------------------------------------ update helpers

@@ -916,12 +916,18 @@ static void launch_stage2d_t(tj_ctx* c, int stage, const MF& in, const MF& base,
                              const Hist& hx, const Hist& hy, const char* nx_name, const char* ny_name) {
     constexpr int TC = TJ_STAGE_TC;
     const Level& lv = c->lv;
-    const UxPlanes ux{c->d_ux, lv.ncells};
+    typename XPart<R>::T x;
     {
         Timed tm(c, nx_name);
-        constexpr int CPW = XGeom<TH>::CPW;
-        const long long waves = (long long)((lv.n[0] + CPW - 1) / CPW) * lv.n[1];
-        hipLaunchKernelGGL((k_xstage<2, TH, R, MX>), dim3(grid1(waves, 4)), dim3(256), 0, c->stream, lv, in, ux, hx, c->d_clk);
+        if constexpr (sizeof(R) == 4) {
+            x = c->Ff[0];
+            const long long waves = (long long)grid1(lv.n[0] + 1, TH ? 61 : 63) * lv.n[1];
+            hipLaunchKernelGGL((k_flux_x<2, TH, R, MX>), dim3(grid1(waves, 4)), dim3(256), 0, c->stream, lv, in, x, hx, c->d_clk);
+        } else {
+            x = UxPlanes{c->d_ux, lv.ncells};
+            const long long waves = (long long)grid1(lv.n[0], XGeom<TH>::CPW) * lv.n[1];
+            hipLaunchKernelGGL((k_xstage<2, TH, MX>), dim3(grid1(waves, 4)), dim3(256), 0, c->stream, lv, in, x, hx, c->d_clk);
+        }
     }
     if (TH) {
         c->pass += 1;
@@ -934,10 +940,10 @@ static void launch_stage2d_t(tj_ctx* c, int stage, const MF& in, const MF& base,
         const long long tiles = (long long)((lv.n[0] + TC - 1) / TC) * ((lv.n[1] + CPW - 1) / CPW);
         if (stage == 1)
             hipLaunchKernelGGL((k_ystage<2, TH, TC, LPS, 1, R, MX>), dim3((unsigned)tiles), dim3(TC * LPS), 0, c->stream, lv,
-                               in, ux, base, out, hy, c->d_clk, ops);
+                               in, x, base, out, hy, c->d_clk, ops);
         else
             hipLaunchKernelGGL((k_ystage<2, TH, TC, LPS, 2, R, MX>), dim3((unsigned)tiles), dim3(TC * LPS), 0, c->stream, lv,
-                               in, ux, base, out, hy, c->d_clk, ops);
+                               in, x, base, out, hy, c->d_clk, ops);
     }
     if (TH) {
         c->pass += 1;

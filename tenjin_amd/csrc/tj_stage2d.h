@@ -1,7 +1,8 @@
 // Stage kernels of two-dimensional fluid levels: one RK stage of
 // HLLCadvance (hllc.cpp:579-695) in two launches, with no face fluxes in HBM.
 //
-//   x kernel  lanes are cells along x (a wave covers one row segment).  MUSCL
+//   x kernel  (FP64; the mixed form's is k_flux_x, see XPart)
+//             lanes are cells along x (a wave covers one row segment).  MUSCL
 //             (+ THINC/BVD) reconstruction, primitiveToConservative and sound
 //             speed of both faces, HLLC at each lane's lower face; then the x
 //             part of update (hllc.cpp:493-523) for each cell whose two faces
@@ -38,6 +39,21 @@ struct UxPlanes {
     double* p;
     long long cs;  // component stride (= cells)
     __device__ __forceinline__ double& at(int q, long long cell) const { return p[(long long)q * cs + cell]; }
+};
+
+// What the y kernel takes the x part of the update from.  FP64: the partial
+// state Ux.  The mixed form, whose stages are bound by HBM, has its x fluxes in
+// FP32 planes (k_flux_x) and adds them in the y kernel: 36 bytes a face written
+// and read in place of 64 a cell, and 116 + 284 (404 in stage 2) bytes a cell
+// in place of 192 + 264 (384); in FP64 the planes would take 72 bytes.  Mixed
+// 2048 x 1024: x 115 -> 94 us, y 135 / 182 -> 140 / 186.
+template <typename R>
+struct XPart {
+    using T = UxPlanes;
+};
+template <>
+struct XPart<float> {
+    using T = FacesT<float>;
 };
 
 // ------------------------------------------------------------------ x kernel
@@ -213,12 +229,12 @@ __device__ __forceinline__ void xstage_body(const Level& lv, const MF& U, const 
     if (st) atomicOr(&clk->status, st);
 }
 
-template <int NM, bool TH, typename R = double, bool MX = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && !MX && sizeof(R) == 8 ? 4 : 1)))
+template <int NM, bool TH, bool MX = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && !MX ? 4 : 1)))
 void k_xstage(Level lv, MF U, UxPlanes Ux, Hist h, Clock* clk) {
     const long long nb = gridDim.x;
     const long long b = xcd_block(blockIdx.x, nb, 2);
-    xstage_body<NM, TH, R, 0, MX>(lv, U, Ux, h, clk, b * (blockDim.x >> 6) + wave_in_block());
+    xstage_body<NM, TH, double, 0, MX>(lv, U, Ux, h, clk, b * (blockDim.x >> 6) + wave_in_block());
 }
 
 // One RK stage of a one-dimensional fluid level in one launch (FIN = STAGE).
@@ -291,7 +307,7 @@ __device__ __forceinline__ void block_min_to_n(double cand, unsigned long long* 
 }
 
 template <int NM, bool TH, int TC, int LPS, int STAGE, typename R, bool MX = false>
-__device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const UxPlanes& Ux, const MF& Ub,
+__device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const typename XPart<R>::T& X, const MF& Ub,
                                             const MF& Uo, const Hist& h, Clock* clk, unsigned ops, long long tile) {
     using T = YTile<NM, TH, TC, LPS, R, MX>;
     constexpr int H = T::H, CPW = T::CPW, NP = T::NP, ROWS = T::ROWS, NF = T::NF, FR = T::FR, NT = T::NT;
@@ -551,18 +567,28 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
         const int cc = e % TC, f = e / TC;
         const int ii = i0 + cc, rr = s0 + f;
         if (ii < nx && rr < ny) {
-            const long long cell = (long long)rr * nx + ii;
             double al[NM], ar[NM], ru[3], E, a0[NM], arl = 0.0;
+            if constexpr (sizeof(R) == 4) {
+                load_cons<NM, MX>(lv, U, ii, rr, 0, al, ar, ru, E, &arl);
 #pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                al[m] = Ux.at(m, cell);
-                ar[m] = Ux.at(NM + m, cell);
-                a0[m] = get_base(U.at(lv.cs[ALPHA] + m, ii, rr, 0));
+                for (int m = 0; m < NM; ++m) a0[m] = al[m];
+                R Fa[NF], Fb[NF];
+                load_faces<NM, R, MX>(X, ii, rr, 0, Fa);
+                load_faces<NM, R, MX>(X, ii + 1, rr, 0, Fb);
+                accum_dir<NM, R, MX>(al, ar, ru, E, a0, dt / lv.dx[0], Fa, Fb, &arl);
+            } else {
+                const long long cell = (long long)rr * nx + ii;
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    al[m] = X.at(m, cell);
+                    ar[m] = X.at(NM + m, cell);
+                    a0[m] = get_base(U.at(lv.cs[ALPHA] + m, ii, rr, 0));
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q) ru[q] = X.at(2 * NM + q, cell);
+                E = X.at(2 * NM + 3, cell);
+                if (MX) arl = X.at(2 * NM + 4, cell);
             }
-#pragma unroll
-            for (int q = 0; q < 3; ++q) ru[q] = Ux.at(2 * NM + q, cell);
-            E = Ux.at(2 * NM + 3, cell);
-            if (MX) arl = Ux.at(2 * NM + 4, cell);
             R Flo[NF], Fhi[NF];
 #pragma unroll
             for (int q = 0; q < NF; ++q) {
@@ -585,11 +611,11 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
 // columns and 16 rows: 264 waves there.
 template <int NM, bool TH, int TC, int LPS, int STAGE, typename R = double, bool MX = false>
 __global__ __launch_bounds__(TC * LPS) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && !MX ? 6 : 1)))
-void k_ystage(Level lv, MF U, UxPlanes Ux, MF Ub, MF Uo, Hist h, Clock* clk, unsigned ops) {
+void k_ystage(Level lv, MF U, typename XPart<R>::T X, MF Ub, MF Uo, Hist h, Clock* clk, unsigned ops) {
     // tiles renumbered per XCD (xcd_block): neighbouring column tiles, which
     // share cache lines of rows whose pitch is not a multiple of the line,
     // and the row bands above and below, which share halo rows, run in one L2
-    ystage_body<NM, TH, TC, LPS, STAGE, R, MX>(lv, U, Ux, Ub, Uo, h, clk, ops, xcd_block(blockIdx.x, gridDim.x, 2));
+    ystage_body<NM, TH, TC, LPS, STAGE, R, MX>(lv, U, X, Ub, Uo, h, clk, ops, xcd_block(blockIdx.x, gridDim.x, 2));
 }
 
 }  // inline namespace TJ_VIEW_NS
