@@ -201,7 +201,8 @@ __global__ __launch_bounds__(256) void k_b_init_p2c(BTab t, int shift) {
 // kernels spread their atomics over them (on one word, the 1365 blocks of a
 // 511^2 problem's stage-2 y kernel serialised to twice the kernel's time).
 // k_b_clock_dt folds and re-arms them before it takes the minimum.
-__global__ __launch_bounds__(64) void k_b_clock_dt(const BProb* P, int np, int driver) {
+// adv: each first ends the step before, as the single level's k_clock_dt.
+__global__ __launch_bounds__(64) void k_b_clock_dt(const BProb* P, int np, int driver, int adv) {
     const int p = blockIdx.x;
     if (p >= np) return;
     Clock* clk = P[p].clk;
@@ -218,33 +219,13 @@ __global__ __launch_bounds__(64) void k_b_clock_dt(const BProb* P, int np, int d
     }
     if (threadIdx.x != 0) return;
     if (b < clk->dtmin_bits) clk->dtmin_bits = b;
-    if (driver) {
-        if (clk->done) return;
-        if (!(clk->t < clk->final_time)) {
-            clk->done = 1;
-            return;
-        }
-    }
-    const double mn = __builtin_bit_cast(double, clk->dtmin_bits);
-    double dt = P[p].lv.cfl * mn;
-    if (driver) {
-        if (clk->t + dt > clk->final_time) dt = clk->final_time - clk->t;
-        if (clk->n < 5) dt *= 0.2;
-    }
-    clk->dt = dt;
-    clk->dtmin_bits = 0x7FEFFFFFFFFFFFFFull;
+    if (adv) clock_advance(clk);
+    clock_dt(clk, P[p].lv.cfl, driver);
 }
 __global__ void k_b_clock_advance(const BProb* P, int np) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
-    Clock* clk = P[p].clk;
-    if (clk->done) return;
-    if (clk->status & ST_STOP) {
-        clk->done = 1;
-        return;
-    }
-    clk->t += clk->dt;
-    clk->n += 1;
+    clock_advance(P[p].clk);
 }
 // zeroes the THINC history planes of every problem in one launch: block
 // row y is problem y, its blocks stride over that problem's planes
@@ -446,14 +427,16 @@ void launch_b_stage2d(tj_batch* b, int g, int stage, unsigned ops) {
     }
 }
 
-// One loop body for every problem: driver dt, two RK stages (the post-step
-// chain fused into stage 2), clock advance.
-int batch_step(tj_batch* b, int prec) {
+// One loop body for every problem: two RK stages (the post-step chain fused
+// into stage 2) between the driver dt and the clock advance.  first: no loop
+// body before it has launched its dt with its advance; next: launch the next
+// one's with this one's advance.
+int batch_step(tj_batch* b, int prec, bool first, bool next) {
     using namespace tj;
     const bool mixed = prec == TJ_PREC_MIXED;
     const unsigned ops = TJ_OP_CLEAN_ALPHA | TJ_OP_DT | TJ_OP_NANCHECK;
     const unsigned gp = grid1(b->np, 64);
-    hipLaunchKernelGGL(k_b_clock_dt, dim3((unsigned)b->np), dim3(64), 0, b->stream, b->d_p, b->np, 1);
+    if (first) hipLaunchKernelGGL(k_b_clock_dt, dim3((unsigned)b->np), dim3(64), 0, b->stream, b->d_p, b->np, 1, 0);
     for (int stage = 1; stage <= 2; ++stage) {
         const int which = stage == 1 ? 0 : 1;
         for (int g = 0; g < 2; ++g) {
@@ -524,7 +507,8 @@ int batch_step(tj_batch* b, int prec) {
             }
         }
     }
-    hipLaunchKernelGGL(k_b_clock_advance, dim3(gp), dim3(64), 0, b->stream, b->d_p, b->np);
+    if (next) hipLaunchKernelGGL(k_b_clock_dt, dim3((unsigned)b->np), dim3(64), 0, b->stream, b->d_p, b->np, 1, 1);
+    else hipLaunchKernelGGL(k_b_clock_advance, dim3(gp), dim3(64), 0, b->stream, b->d_p, b->np);
     BHIPCHK(b, hipGetLastError());
     return TJ_OK;
 }
@@ -714,7 +698,7 @@ int tj_batch_advance(tj_batch* b, int nsteps, int prec) {
     }
     int r;
     for (int q = 0; q < nsteps; ++q)
-        if ((r = batch_step(b, prec))) return r;
+        if ((r = batch_step(b, prec, q == 0, q + 1 < nsteps))) return r;
     return TJ_OK;
 }
 

@@ -29,6 +29,36 @@ __device__ __forceinline__ unsigned long long* dt_slot(const Level& lv, Clock* c
     return lv.dtpart ? lv.dtpart + (blockIdx.x % DT_PARTS) : &clk->dtmin_bits;
 }
 
+// End of a loop iteration: the NaN stop of main.cpp:183-187 (before t, n
+// advance), else t += dt, n++ (main.cpp:121).  One thread.
+__device__ __forceinline__ void clock_advance(Clock* clk) {
+    if (clk->done) return;
+    if (atomicOr(&clk->status, 0u) & ST_STOP) {
+        clk->done = 1;
+        return;
+    }
+    clk->t += clk->dt;
+    clk->n += 1;
+}
+// The next dt from the folded minimum (k_clock_dt).  One thread.
+__device__ __forceinline__ void clock_dt(Clock* clk, double cfl, int driver) {
+    if (driver) {
+        if (clk->done) return;
+        if (!(clk->t < clk->final_time)) {
+            clk->done = 1;
+            return;
+        }
+    }
+    const double mn = __builtin_bit_cast(double, clk->dtmin_bits);
+    double dt = cfl * mn;
+    if (driver) {
+        if (clk->t + dt > clk->final_time) dt = clk->final_time - clk->t;
+        if (clk->n < 5) dt *= 0.2;
+    }
+    clk->dt = dt;
+    clk->dtmin_bits = DT_NONE;
+}
+
 // Everything below takes or launches with the state view MF (see tj_device.h).
 inline namespace TJ_VIEW_NS {
 
@@ -809,8 +839,10 @@ __global__ __launch_bounds__(256) void k_sound_dt(Level lv, MF U, Clock* clk) {
 // dt = CFL * min (timestep.cpp:61-69); with `driver` the loop test and the
 // clamps of main.cpp:121, 135-143.  Re-arms the min word and, with `part`
 // (DT_PARTS words, launched with one wave), first folds the partial slots
-// into it and re-arms them.
-__global__ void k_clock_dt(Clock* clk, double cfl, int driver, unsigned long long* part) {
+// into it and re-arms them.  With `adv` it first ends the step before
+// (k_clock_advance): between two steps of a run the two are one launch (four
+// steps of three 701 x 389 levels at once 304 -> 300 us each).
+__global__ void k_clock_dt(Clock* clk, double cfl, int driver, unsigned long long* part, int adv) {
     if (blockIdx.x != 0) return;
     if (part) {
         unsigned long long b = DT_NONE;
@@ -826,37 +858,16 @@ __global__ void k_clock_dt(Clock* clk, double cfl, int driver, unsigned long lon
         if (threadIdx.x == 0 && b < clk->dtmin_bits) clk->dtmin_bits = b;
     }
     if (threadIdx.x != 0) return;
-    if (driver) {
-        if (clk->done) return;
-        if (!(clk->t < clk->final_time)) {
-            clk->done = 1;
-            return;
-        }
-    }
-    const double mn = __builtin_bit_cast(double, clk->dtmin_bits);
-    double dt = cfl * mn;
-    if (driver) {
-        if (clk->t + dt > clk->final_time) dt = clk->final_time - clk->t;
-        if (clk->n < 5) dt *= 0.2;
-    }
-    clk->dt = dt;
-    clk->dtmin_bits = DT_NONE;
+    if (adv) clock_advance(clk);
+    clock_dt(clk, cfl, driver);
 }
 // fill of the partial CFL slots with the empty value
 __global__ void k_dtpart_reset(unsigned long long* part) {
     for (int q = (int)threadIdx.x; q < DT_PARTS; q += (int)blockDim.x) part[q] = DT_NONE;
 }
-// end of a loop iteration: the NaN stop of main.cpp:183-187 (before t, n
-// advance), else t += dt, n++ (main.cpp:121).
 __global__ void k_clock_advance(Clock* clk) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (clk->done) return;
-    if (clk->status & ST_STOP) {
-        clk->done = 1;
-        return;
-    }
-    clk->t += clk->dt;
-    clk->n += 1;
+    clock_advance(clk);
 }
 __global__ void k_clock_final(Clock* clk, double final_time) {
     if (threadIdx.x == 0 && blockIdx.x == 0) clk->final_time = final_time;

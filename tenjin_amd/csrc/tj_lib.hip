@@ -583,7 +583,7 @@ int tj_compute_dt(tj_ctx* c, const tj_mf* U, double* dt_out) {
     if (r) return r;
     HIPCHK(c, hipSetDevice(c->device));
     launch_sound_dt(c, view(U));
-    hipLaunchKernelGGL(k_clock_dt, dim3(1), dim3(64), 0, c->stream, c->d_clk, c->lv.cfl, 0, c->d_dtpart);
+    hipLaunchKernelGGL(k_clock_dt, dim3(1), dim3(64), 0, c->stream, c->d_clk, c->lv.cfl, 0, c->d_dtpart, 0);
     HIPCHK(c, hipGetLastError());
     if (dt_out) {
         Clock h;
@@ -629,7 +629,7 @@ int tj_get_clock(tj_ctx* c, double* t, double* dt, int* n) {
 int tj_driver_dt(tj_ctx* c, double final_time) {
     if (!c || !c->bound) return TJ_ENOLEVEL;
     hipLaunchKernelGGL(k_clock_final, dim3(1), dim3(64), 0, c->stream, c->d_clk, final_time);
-    hipLaunchKernelGGL(k_clock_dt, dim3(1), dim3(64), 0, c->stream, c->d_clk, c->lv.cfl, 1, c->d_dtpart);
+    hipLaunchKernelGGL(k_clock_dt, dim3(1), dim3(64), 0, c->stream, c->d_clk, c->lv.cfl, 1, c->d_dtpart, 0);
     HIPCHK(c, hipGetLastError());
     return TJ_OK;
 }
@@ -985,14 +985,15 @@ static int launch_stage2d(tj_ctx* c, int stage, const MF& in, const MF& base, co
 static bool use_stage2d(const tj_ctx* c) { return c->stage2d && c->d_ux && stage2d_level(c); }
 
 // One-dimensional fluid levels without a mixture: each RK stage is one launch
-// of k_xstage1d (the x stage completing its cells); with `tail` stage 2 also
-// advances the clock (k_clock_advance's work).
+// of k_xstage1d (the x stage completing its cells); with `tail` 1 stage 2 also
+// advances the clock (k_clock_advance's work), with 2 it also takes the next
+// step's dt (k_clock_dt's).
 static bool use_stage1d(const tj_ctx* c) {
     return c->stage2d && c->d_ticket && !c->lv.solid && c->lv.dim == 1 && c->lv.mixm < 0;
 }
 extern "C++" {
 template <bool TH, typename R>
-static void launch_stage1d_t(tj_ctx* c, int stage, const MF& in, const MF& base, const MF& out, unsigned ops, bool tail,
+static void launch_stage1d_t(tj_ctx* c, int stage, const MF& in, const MF& base, const MF& out, unsigned ops, int tail,
                              const char* name) {
     const Level& lv = c->lv;
     const Hist h = hist_for(c, 0);
@@ -1002,13 +1003,13 @@ static void launch_stage1d_t(tj_ctx* c, int stage, const MF& in, const MF& base,
         const unsigned g = grid1((long long)((lv.n[0] + CPW - 1) / CPW) * lv.n[1], 4);
         if (stage == 1)
             hipLaunchKernelGGL((k_xstage1d<2, TH, 1, false, R>), dim3(g), dim3(256), 0, c->stream, lv, in, base, out, h,
-                               c->d_clk, ops, c->d_ticket);
+                               c->d_clk, ops, c->d_ticket, tail == 2);
         else if (tail)
             hipLaunchKernelGGL((k_xstage1d<2, TH, 2, true, R>), dim3(g), dim3(256), 0, c->stream, lv, in, base, out, h,
-                               c->d_clk, ops, c->d_ticket);
+                               c->d_clk, ops, c->d_ticket, tail == 2);
         else
             hipLaunchKernelGGL((k_xstage1d<2, TH, 2, false, R>), dim3(g), dim3(256), 0, c->stream, lv, in, base, out, h,
-                               c->d_clk, ops, c->d_ticket);
+                               c->d_clk, ops, c->d_ticket, tail == 2);
     }
     if (TH) {
         c->pass += 1;
@@ -1016,7 +1017,7 @@ static void launch_stage1d_t(tj_ctx* c, int stage, const MF& in, const MF& base,
     }
 }
 }  // extern "C++"
-static int launch_stage1d(tj_ctx* c, int stage, const MF& in, const MF& base, const MF& out, unsigned ops, bool tail,
+static int launch_stage1d(tj_ctx* c, int stage, const MF& in, const MF& base, const MF& out, unsigned ops, int tail,
                           int prec) {
     const bool mixed = prec == TJ_PREC_MIXED;
     static const char* nm[2][2] = {{"xstage1d_1", "xstage1d_2_post"}, {"xstage1d_1_mixed", "xstage1d_2_post_mixed"}};
@@ -1057,7 +1058,7 @@ int tj_rk_stage(tj_ctx* c, int stage, const tj_mf* Uin, const tj_mf* Ubase, tj_m
     // Uout: an in-place stage (Uout == Uin) takes the flux-plane passes
     if (use_stage2d(c) && !same_view(view(Uout), in)) return launch_stage2d(c, stage, in, base, view(Uout), 0u, prec);
     if (stage == 1 && use_stage1_solid(c) && !same_view(view(Uout), in)) return launch_stage1_solid(c, in, view(Uout), prec);
-    if (use_stage1d(c) && !same_view(view(Uout), in)) return launch_stage1d(c, stage, in, base, view(Uout), 0u, false, prec);
+    if (use_stage1d(c) && !same_view(view(Uout), in)) return launch_stage1d(c, stage, in, base, view(Uout), 0u, 0, prec);
     const FuseArgs fz{stage, base, view(Uout), 0u};
     bool fused = false;
     if ((r = launch_fluxes(c, in, &fz, &fused, prec))) return r;
@@ -1108,9 +1109,14 @@ int tj_post_step(tj_ctx* c, tj_mf* U, unsigned ops) {
     return TJ_OK;
 }
 
-int tj_step(tj_ctx* c, tj_mf* S, tj_mf* T, int prec) {
-    if (!c || !c->bound) return TJ_ENOLEVEL;
-    TJ_FORWARD_FABS(c, tj_step(c, S, T, prec), S, T);
+// The end of a step: the clock's advance, and between two steps of a run the
+// next driver dt in the same launch.
+static void launch_step_end(tj_ctx* c, bool next) {
+    if (next) hipLaunchKernelGGL(k_clock_dt, dim3(1), dim3(64), 0, c->stream, c->d_clk, c->lv.cfl, 1, c->d_dtpart, 1);
+    else hipLaunchKernelGGL(k_clock_advance, dim3(1), dim3(64), 0, c->stream, c->d_clk);
+}
+// Both stages with the clock's dt, then the step's end.
+static int run_step(tj_ctx* c, tj_mf* S, tj_mf* T, int prec, bool next) {
     int r;
     if ((r = check_prec(c, prec))) return r;
     if ((r = check_mf(c, S)) || (r = check_mf(c, T))) return r;
@@ -1121,13 +1127,13 @@ int tj_step(tj_ctx* c, tj_mf* S, tj_mf* T, int prec) {
     if (use_stage2d(c)) {
         if ((r = launch_stage2d(c, 1, s, s, t, 0u, prec))) return r;
         if ((r = launch_stage2d(c, 2, t, s, s, step_ops(c), prec))) return r;
-        hipLaunchKernelGGL(k_clock_advance, dim3(1), dim3(64), 0, c->stream, c->d_clk);
+        launch_step_end(c, next);
         HIPCHK(c, hipGetLastError());
         return TJ_OK;
     }
-    if (use_stage1d(c)) {  // two launches; the second advances the clock
-        if ((r = launch_stage1d(c, 1, s, s, t, 0u, false, prec))) return r;
-        return launch_stage1d(c, 2, t, s, s, step_ops(c), true, prec);
+    if (use_stage1d(c)) {  // two launches; the second ends the step
+        if ((r = launch_stage1d(c, 1, s, s, t, 0u, 0, prec))) return r;
+        return launch_stage1d(c, 2, t, s, s, step_ops(c), next ? 2 : 1, prec);
     }
     bool fused = false;
     const FuseArgs f1{1, s, t, 0u};
@@ -1146,9 +1152,15 @@ int tj_step(tj_ctx* c, tj_mf* S, tj_mf* T, int prec) {
         Timed tm(c, mixed ? "update_stage2_post_mixed" : "update_stage2_post");
         launch_update(c, 2, t, s, s, step_ops(c), prec);
     }
-    hipLaunchKernelGGL(k_clock_advance, dim3(1), dim3(64), 0, c->stream, c->d_clk);
+    launch_step_end(c, next);
     HIPCHK(c, hipGetLastError());
     return TJ_OK;
+}
+
+int tj_step(tj_ctx* c, tj_mf* S, tj_mf* T, int prec) {
+    if (!c || !c->bound) return TJ_ENOLEVEL;
+    TJ_FORWARD_FABS(c, tj_step(c, S, T, prec), S, T);
+    return run_step(c, S, T, prec, false);
 }
 
 int tj_begin_run(tj_ctx* c, const tj_mf* S, double final_time) {
@@ -1169,8 +1181,8 @@ int tj_advance_steps(tj_ctx* c, tj_mf* S, tj_mf* T, int nsteps, int prec) {
     TJ_FORWARD_FABS(c, tj_advance_steps(c, S, T, nsteps, prec), S, T);
     int r;
     for (int q = 0; q < nsteps; ++q) {
-        hipLaunchKernelGGL(k_clock_dt, dim3(1), dim3(64), 0, c->stream, c->d_clk, c->lv.cfl, 1, c->d_dtpart);
-        if ((r = TJ_SELF(tj_step)(c, S, T, prec))) return r;
+        if (q == 0) hipLaunchKernelGGL(k_clock_dt, dim3(1), dim3(64), 0, c->stream, c->d_clk, c->lv.cfl, 1, c->d_dtpart, 0);
+        if ((r = run_step(c, S, T, prec, q + 1 < nsteps))) return r;
     }
     return TJ_OK;
 }
