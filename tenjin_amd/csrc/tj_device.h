@@ -55,8 +55,8 @@ struct Level {
     int cs[NVAR];      // first component of each Variable (AccessPattern), -1 if absent
     long long ncells;
     int mixm;          // the mixture material (MixtureEOS), -1 if none
-    // materials with derivative parts (MatT<Dual<K>>[MAXM], device memory) for
-    // the tangent-linear form; null elsewhere
+    // materials with derivative parts (MatT<Dual<K>>[MAXM] per direction group,
+    // device memory) for the tangent-linear form; null elsewhere
     const void* md;
     // partial slots of the CFL minimum (DT_PARTS words; null: the clock's word)
     unsigned long long* dtpart;
@@ -64,7 +64,7 @@ struct Level {
 
 template <typename R>
 __device__ __forceinline__ const MatT<R>& mat(const Level& lv, int m) {
-    return static_cast<const MatT<R>*>(lv.md)[m];
+    return static_cast<const MatT<R>*>(lv.md)[blockIdx.y * MAXM + m];  // grid row y: direction group y
 }
 template <>
 __device__ __forceinline__ const MatT<double>& mat<double>(const Level& lv, int m) { return lv.m[m]; }

@@ -12,6 +12,13 @@
 // planes hold the NF flux components of the values, then NF per direction.
 // The time step is differentiated through dt = CFL min(dx / (a + |u|)) along
 // the cell that attains the minimum (the lowest cell index on ties).
+//
+// Grid row y of every launch runs direction group y: its own values,
+// derivatives, faces, history planes, materials and clock, one after the other
+// in each buffer.  A level of 160^2 cells gives 480 waves a launch, half of the
+// 1024 that the kernels hold at one wave per SIMD, so its groups run side by
+// side (three groups of two directions, eight steps: 7840 -> 5055 us); a level
+// that fills the device alone has one row at a time.
 #pragma once
 #include "tj_dual.h"
 #include "tj_solid_kernels.h"
@@ -23,6 +30,13 @@ struct DMF {
     MF u;           // values
     MF dd;          // derivative block 0 (compact strides)
     long long bs;   // stride between derivative blocks
+    long long gu, gd;  // strides between direction groups of the values and the derivatives
+    __device__ __forceinline__ DMF row() const {  // this grid row's group
+        DMF r = *this;
+        r.u.p += (long long)blockIdx.y * gu;
+        r.dd.p += (long long)blockIdx.y * gd;
+        return r;
+    }
     __device__ __forceinline__ Dual<K> get(int c, int i, int j, int k) const {
         Dual<K> x;
         x.v = u.at(c, i, j, k);
@@ -93,7 +107,10 @@ __device__ __forceinline__ void load_tprim(const Level& lv, const DMF<K>& U, int
 // built, so two face states are live at a time.
 template <int NM, int K, int D>
 __global__ __launch_bounds__(256) void k_tflux_ts(Level lv, DMF<K> U, Faces F, Clock* clk) {
+    clk += blockIdx.y;
     if (clk->done) return;
+    U = U.row();
+    F.p += blockIdx.y * (3 * NM + 17) * (K + 1) * F.cs;
     constexpr int LN = D == 0 ? 64 : 8;  // lanes along D
     constexpr int LT = 64 / LN;           // lanes along x (D = 1, 2)
     constexpr int PER = LN - 1;           // faces per tile column
@@ -230,7 +247,16 @@ __device__ __forceinline__ double tsound_cand(const Level& lv, const DMF<K>& U, 
 template <int NM, int STAGE, int K>
 __global__ __launch_bounds__(256) void k_tupdate_s(Level lv, DMF<K> Uin, DMF<K> Ub, DMF<K> Uo, Faces F0, Faces F1,
                                                    Faces F2, Clock* clk, const double* tdt, unsigned ops, double* cand) {
+    clk += blockIdx.y;
     if (clk->done) return;
+    Uin = Uin.row();
+    Ub = Ub.row();
+    Uo = Uo.row();
+    F0.p += blockIdx.y * (3 * NM + 17) * (K + 1) * F0.cs;
+    F1.p += blockIdx.y * (3 * NM + 17) * (K + 1) * F1.cs;
+    F2.p += blockIdx.y * (3 * NM + 17) * (K + 1) * F2.cs;
+    tdt += blockIdx.y * (K + 1);
+    cand += blockIdx.y * (K + 1) * lv.ncells;
     using T = Dual<K>;
     constexpr int NC = 3 * NM + 13, NF = NC + 4;
     const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
@@ -352,6 +378,9 @@ __global__ __launch_bounds__(256) void k_tupdate_s(Level lv, DMF<K> Uin, DMF<K> 
 // getTimeStep of a state (k_sound_dt_s) with the candidates' derivatives.
 template <int NM, int K>
 __global__ __launch_bounds__(256) void k_tsound_dt_s(Level lv, DMF<K> U, Clock* clk, double* cand) {
+    clk += blockIdx.y;
+    U = U.row();
+    cand += blockIdx.y * (K + 1) * lv.ncells;
     const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     double cv = __builtin_huge_val();
@@ -371,6 +400,7 @@ __global__ __launch_bounds__(256) void k_tsound_dt_s(Level lv, DMF<K> U, Clock* 
 // EOS parameters through the materials' derivative parts.
 template <int NM, int K>
 __global__ __launch_bounds__(256) void k_tinit_p2c_s(Level lv, DMF<K> U, int shift) {
+    U = U.row();
     using T = Dual<K>;
     const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -417,8 +447,12 @@ __global__ __launch_bounds__(256) void k_tinit_p2c_s(Level lv, DMF<K> U, int shi
 }
 
 // The lowest cell index whose candidate attains the level minimum.
+// cstride: between the candidates of two direction groups.
 __global__ __launch_bounds__(256) void k_targmin(const Clock* clk, const double* cand, long long ncell,
-                                                 unsigned long long* arg) {
+                                                 unsigned long long* arg, long long cstride) {
+    clk += blockIdx.y;
+    cand += blockIdx.y * cstride;
+    arg += blockIdx.y;
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (id < ncell && __builtin_bit_cast(unsigned long long, cand[id]) == clk->dtmin_bits)
         atomicMin(arg, (unsigned long long)id);
@@ -431,6 +465,11 @@ template <int K>
 __global__ void k_tclock_dt(Clock* clk, double cfl, const double* cand, long long ncell, unsigned long long* arg,
                             double* tdt, const double* tt) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    clk += blockIdx.y;
+    cand += blockIdx.y * (K + 1) * ncell;
+    arg += blockIdx.y;
+    tdt += blockIdx.y * (K + 1);
+    tt += blockIdx.y * K;
     if (clk->done) return;
     if (!(clk->t < clk->final_time)) {
         clk->done = 1;
@@ -459,11 +498,16 @@ __global__ void k_tclock_dt(Clock* clk, double cfl, const double* cand, long lon
     clk->dtmin_bits = 0x7FEFFFFFFFFFFFFFull;
     *arg = ~0ull;
 }
-// start of a run (k_clock_final of tj_begin_run): the final time, no
-// minimising cell yet, t's derivatives zero
+// start of a run (k_clock_final of tj_begin_run): the level's clock c0 as
+// tj_set_dt left it, the final time, no minimising cell yet, t's derivatives
+// zero
 template <int K>
-__global__ void k_tclock_begin(Clock* clk, double final_time, unsigned long long* arg, double* tt) {
+__global__ void k_tclock_begin(Clock* clk, const Clock* c0, double final_time, unsigned long long* arg, double* tt) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    clk += blockIdx.y;
+    arg += blockIdx.y;
+    tt += blockIdx.y * K;
+    if (clk != c0) *clk = *c0;
     clk->final_time = final_time;
     *arg = ~0ull;
 #pragma unroll
@@ -473,6 +517,9 @@ __global__ void k_tclock_begin(Clock* clk, double final_time, unsigned long long
 template <int K>
 __global__ void k_tclock_advance(Clock* clk, const double* tdt, double* tt) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    clk += blockIdx.y;
+    tdt += blockIdx.y * (K + 1);
+    tt += blockIdx.y * K;
     if (clk->done) return;
     if (clk->status & ST_STOP) {
         clk->done = 1;
@@ -501,6 +548,16 @@ struct THist {
     double* edge_out;
     long long pstride, estride;  // plane strides (cells, faces of the direction)
     long long pblk, eblk;        // derivative block strides (NM planes)
+    __device__ __forceinline__ THist row(int K) const {  // this grid row's direction group
+        THist r = *this;
+        const long long p = blockIdx.y * (K + 1) * pblk, e = blockIdx.y * (K + 1) * eblk;
+        r.urstar += p;
+        r.star_in += p;
+        r.star_out += p;
+        r.edge_in += e;
+        r.edge_out += e;
+        return r;
+    }
 };
 template <int K>
 __device__ __forceinline__ Dual<K> hget(const double* p, long long blk, long long idx) {
@@ -570,7 +627,11 @@ __device__ __forceinline__ FSt<NM, Dual<K>> shfl_tfst(const FSt<NM, Dual<K>>& S,
 // written only where it is, so the writes race with no read.
 template <int NM, int K, int D, bool TH>
 __global__ __launch_bounds__(256) void k_tflux_tf(Level lv, DMF<K> U, Faces F, THist h, Clock* clk) {
+    clk += blockIdx.y;
     if (clk->done) return;
+    U = U.row();
+    F.p += blockIdx.y * (2 * NM + 5) * (K + 1) * F.cs;
+    if (TH) h = h.row(K);
     constexpr int LN = D == 0 ? 64 : 8;  // lanes along D
     constexpr int LT = 64 / LN;           // lanes along x (D = 1, 2)
     constexpr int PER = LN - 1;           // faces per tile column
@@ -755,7 +816,16 @@ __device__ __forceinline__ double tcand_f(const Level& lv, const DMF<K>& U, Dual
 template <int NM, int STAGE, int K>
 __global__ __launch_bounds__(256) void k_tupdate_f(Level lv, DMF<K> Uin, DMF<K> Ub, DMF<K> Uo, Faces F0, Faces F1,
                                                    Faces F2, Clock* clk, const double* tdt, unsigned ops, double* cand) {
+    clk += blockIdx.y;
     if (clk->done) return;
+    Uin = Uin.row();
+    Ub = Ub.row();
+    Uo = Uo.row();
+    F0.p += blockIdx.y * (2 * NM + 5) * (K + 1) * F0.cs;
+    F1.p += blockIdx.y * (2 * NM + 5) * (K + 1) * F1.cs;
+    F2.p += blockIdx.y * (2 * NM + 5) * (K + 1) * F2.cs;
+    tdt += blockIdx.y * (K + 1);
+    cand += blockIdx.y * (K + 1) * lv.ncells;
     using T = Dual<K>;
     constexpr int NF = 2 * NM + 5;
     const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
@@ -860,6 +930,9 @@ __global__ __launch_bounds__(256) void k_tupdate_f(Level lv, DMF<K> Uin, DMF<K> 
 
 template <int NM, int K>
 __global__ __launch_bounds__(256) void k_tsound_dt_f(Level lv, DMF<K> U, Clock* clk, double* cand) {
+    clk += blockIdx.y;
+    U = U.row();
+    cand += blockIdx.y * (K + 1) * lv.ncells;
     using T = Dual<K>;
     const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -885,6 +958,7 @@ __global__ __launch_bounds__(256) void k_tsound_dt_f(Level lv, DMF<K> U, Clock* 
 
 template <int NM, int K>
 __global__ __launch_bounds__(256) void k_tinit_p2c_f(Level lv, DMF<K> U, int shift) {
+    U = U.row();
     using T = Dual<K>;
     const int nx = lv.n[0], ny = lv.n[1], nz = lv.n[2];
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -933,8 +1007,10 @@ __global__ __launch_bounds__(256) void k_copy_mf(MF X, MF Z, int ncomp, int nx, 
 }
 // value and derivatives of one component of one cell into a trace row
 template <int K>
-__global__ void k_tprobe(DMF<K> U, int c, int i, int j, int k, double* row) {
+__global__ void k_tprobe(DMF<K> U, int c, int i, int j, int k, double* row, long long rstride) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    U = U.row();
+    row += blockIdx.y * rstride;
     const Dual<K> x = U.get(c, i, j, k);
     row[0] = x.v;
 #pragma unroll
