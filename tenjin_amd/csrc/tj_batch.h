@@ -167,6 +167,34 @@ void k_b_xstage1d(BTab t, int q, int e, unsigned ops) {
     if (STAGE == 1) xstage_body<2, TH, R, 1>(P.lv, P.S, UxPlanes{}, bhist(P, 0, q, e), P.clk, w, XFin{P.S, P.T, ops});
     else xstage_body<2, TH, R, 2>(P.lv, P.T, UxPlanes{}, bhist(P, 0, q, e), P.clk, w, XFin{P.S, P.S, ops});
 }
+// The 1D problems' stage and the 2D problems' x part in one launch: the first
+// b1 blocks are k_b_xstage1d's, whose few waves (1D problems hold 1 % of an
+// ensemble's cells) would leave the device idle for 16 to 20 us a stage, the
+// others k_b_flux_x's or k_b_xstage's (16 tubes and 16 squares: mixed 649 ->
+// 628 us a step, FP64 730 -> 700).
+template <bool TH, int STAGE, typename R>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && sizeof(R) == 8 ? 4 : 1)))
+void k_b_x12(BTab t1, int q1, int e1, unsigned ops, unsigned b1, BTab t2, int q2, int e2) {
+    if (blockIdx.x < b1) {
+        const long long gw = bwave();
+        if (gw >= bunits(t1)) return;
+        const int p = bfind(t1.start, t1.np, gw);
+        const BProb& P = ro_at(t1.p, p);
+        const long long w = gw - ro_at(t1.start, p);
+        const XFin fin = STAGE == 1 ? XFin{P.S, P.T, ops} : XFin{P.S, P.S, ops};
+        xstage_body<2, TH, R, STAGE>(P.lv, STAGE == 1 ? P.S : P.T, UxPlanes{}, bhist(P, 0, q1, e1), P.clk, w, fin);
+    } else {
+        const long long gw = xcd_block(blockIdx.x - b1, gridDim.x - b1, 2) * (blockDim.x >> 6) + wave_in_block();
+        if (gw >= bunits(t2)) return;
+        const int p = bfind(t2.start, t2.np, gw);
+        const BProb& P = ro_at(t2.p, p);
+        const long long w = gw - ro_at(t2.start, p);
+        if constexpr (sizeof(R) == 4)
+            flux_x_body<2, TH, R>(P.lv, STAGE == 1 ? P.S : P.T, P.Ff[0], bhist(P, 0, q2, e2), P.clk, w);
+        else
+            xstage_body<2, TH, R>(P.lv, STAGE == 1 ? P.S : P.T, P.ux, bhist(P, 0, q2, e2), P.clk, w);
+    }
+}
 template <bool TH, int TC, int LPS, int STAGE, typename R>
 __global__ __launch_bounds__(TC * LPS) void k_b_ystage(BTab t, int q, int e, unsigned ops) {
     const long long gb = xcd_block(blockIdx.x, gridDim.x, 2);  // as k_ystage
@@ -380,19 +408,35 @@ void batch_clear_graph(tj_batch* b) {
     b->graph = nullptr;
 }
 
-// The stage kernels of group g (2D): x stage, then y stage per tile shape.
+// The stage kernels of group 1 (2D): x stage, with the 1D problems' stage in
+// the same launch where there are any, then y stage per tile shape.
 template <bool TH, typename R>
-void launch_b_stage2d(tj_batch* b, int g, int stage, unsigned ops) {
+void launch_b_stage2d(tj_batch* b, int stage, unsigned ops) {
     using namespace tj;
+    constexpr int g = 1;
     const int which = stage == 1 ? 0 : 1;
     {
         const int q = (int)(b->pass[g] & 1), e = (int)(b->dpass[g][0] & 1);
-        if constexpr (sizeof(R) == 4)
-            hipLaunchKernelGGL((k_b_flux_x<TH, R>), dim3(grid1(b->tot[g][0], 4)), dim3(256), 0, b->stream, tab(b, g, 0),
-                               which, q, e);
-        else
-            hipLaunchKernelGGL((k_b_xstage<TH>), dim3(grid1(b->tot[g][3], 4)), dim3(256), 0, b->stream, tab(b, g, 3),
-                               which, q, e);
+        const BTab tx = tab(b, g, sizeof(R) == 4 ? 0 : 3);
+        const unsigned gx = grid1(b->tot[g][sizeof(R) == 4 ? 0 : 3], 4);
+        if (b->tot[0][2] != 0) {
+            const int q1 = (int)(b->pass[0] & 1), e1 = (int)(b->dpass[0][0] & 1);
+            const unsigned g1 = grid1(b->tot[0][3], 4);
+            if (stage == 1)
+                hipLaunchKernelGGL((k_b_x12<TH, 1, R>), dim3(g1 + gx), dim3(256), 0, b->stream, tab(b, 0, 3), q1, e1, 0u, g1,
+                                   tx, q, e);
+            else
+                hipLaunchKernelGGL((k_b_x12<TH, 2, R>), dim3(g1 + gx), dim3(256), 0, b->stream, tab(b, 0, 3), q1, e1, ops, g1,
+                                   tx, q, e);
+            if (b->thinc) {
+                b->pass[0] += 1;
+                b->dpass[0][0] += 1;
+            }
+        } else if constexpr (sizeof(R) == 4) {
+            hipLaunchKernelGGL((k_b_flux_x<TH, R>), dim3(gx), dim3(256), 0, b->stream, tx, which, q, e);
+        } else {
+            hipLaunchKernelGGL((k_b_xstage<TH>), dim3(gx), dim3(256), 0, b->stream, tx, which, q, e);
+        }
         if (b->thinc) {
             b->pass[g] += 1;
             b->dpass[g][0] += 1;
@@ -442,12 +486,13 @@ int batch_step(tj_batch* b, int prec, bool first, bool next) {
         for (int g = 0; g < 2; ++g) {
             if (b->tot[g][2] == 0) continue;
             if (g == 1 && b->stage2d) {
-                if (b->thinc && mixed) launch_b_stage2d<true, float>(b, g, stage, ops);
-                else if (b->thinc) launch_b_stage2d<true, double>(b, g, stage, ops);
-                else if (mixed) launch_b_stage2d<false, float>(b, g, stage, ops);
-                else launch_b_stage2d<false, double>(b, g, stage, ops);
+                if (b->thinc && mixed) launch_b_stage2d<true, float>(b, stage, ops);
+                else if (b->thinc) launch_b_stage2d<true, double>(b, stage, ops);
+                else if (mixed) launch_b_stage2d<false, float>(b, stage, ops);
+                else launch_b_stage2d<false, double>(b, stage, ops);
                 continue;
             }
+            if (g == 0 && b->stage2d && b->tot[1][2] != 0) continue;  // in the 2D problems' x launch
             if (g == 0 && b->stage2d) {  // 1D problems: one launch per stage, no flux planes
                 const int q = (int)(b->pass[g] & 1), e = (int)(b->dpass[g][0] & 1);
                 const unsigned gx = grid1(b->tot[g][3], 4);
