@@ -34,6 +34,7 @@ struct tj_ctx {
     double* d_estar[3][2] = {{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}};
     long long estride[3] = {0, 0, 0};
     Clock* d_clk = nullptr;
+    double* h_dt = nullptr;  // pinned word for tj_compute_dt's result (null: pageable)
     unsigned long long* d_dtpart = nullptr;  // DT_PARTS partial slots of the CFL minimum
     unsigned* d_ticket = nullptr;            // wave tickets of the one-launch 1D stage (k_xstage1d), 0 between launches
     unsigned* d_status = nullptr;

@@ -869,6 +869,21 @@ __global__ void k_clock_advance(Clock* clk) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     clock_advance(clk);
 }
+// tj_set_dt: the dt of the next step, and with `reset` the start of a loop
+// (the partial CFL slots emptied with it; launched with one wave)
+__global__ void k_clock_set(Clock* clk, double dt, int reset, unsigned long long* part) {
+    if (reset && part)
+        for (int q = (int)threadIdx.x; q < DT_PARTS; q += (int)blockDim.x) part[q] = DT_NONE;
+    if (threadIdx.x != 0) return;
+    clk->dt = dt;
+    if (!reset) return;
+    clk->t = 0.0;
+    clk->n = 0;
+    clk->done = 0;
+    clk->status = 0;
+    clk->final_time = __builtin_huge_val();
+    clk->dtmin_bits = DT_NONE;
+}
 __global__ void k_clock_final(Clock* clk, double final_time) {
     if (threadIdx.x == 0 && blockIdx.x == 0) clk->final_time = final_time;
 }
