@@ -47,6 +47,41 @@ def test_mixture_stage_tiles_match_oracle(nx, ny, thinc):
     assert g.status() == f.status() == o.status()
 
 
+@pytest.mark.parametrize("seed,energy", [(1, 0.0), (2, 0.5), (3, 4.0)])
+def test_bisection_signs_match_oracle(seed, energy):
+    """rootFind's known signs: cells whose mass fraction, density, pressure and
+    (for energy > 0) total energy are drawn over decades, brackets without a
+    sign change among them, against the oracle's plain bisection, bit for bit."""
+    from oracle.oracle import Oracle
+    from tenjin_amd import GpuLevel
+    from tenjin_amd.configs import ALPHA, ALPHARHO, LAMBDA, P, RHO_K, TOTAL_E
+
+    rng = np.random.default_rng(seed)
+    pb = _tube(37, 29, 0)
+    L, U, shape = pb.layout, pb.prims.copy(), pb.prims.shape[1:]
+    al = 10.0 ** rng.uniform(-6.0, 0.0, shape)
+    print(f"\n[case] bisection seed {seed} energy {energy}", flush=True)
+    for m in range(2):
+        U[L.comp(ALPHA, m)] = (al, 1.0 - al)[m]
+        U[L.comp(RHO_K, m)] = 10.0 ** rng.uniform(0.0, 3.8, shape)
+    U[L.comp(LAMBDA)] = rng.uniform(0.0, 1.0, shape)
+    U[L.comp(P)] = 10.0 ** rng.uniform(4.0, 11.0, shape)
+    pb = dataclasses.replace(pb, prims=U)
+    o, g = Oracle(pb), GpuLevel(pb)
+    g.init_from_prims(pb.prims)
+    s = o.get()
+    assert np.array_equal(s[L.comp(ALPHARHO)], g.get_state()[L.comp(ALPHARHO)])
+    s[L.comp(TOTAL_E)] *= 10.0 ** (energy * rng.uniform(-1.0, 1.0, shape))
+    o.set(s)
+    g.set_state(s)
+    o.c2p()
+    g.c2p()
+    ref, got = o.get(), g.get_state()
+    for c in L.state_comps():
+        assert np.array_equal(ref[c], got[c], equal_nan=True), L.names[c]
+    assert g.status() == o.status()
+
+
 def test_static_scratch_without_stage_planes():
     import torch
 
