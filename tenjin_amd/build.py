@@ -5,8 +5,9 @@ the source tree), the C++ host interface tenjin_amd/csrc/host/ into
 tenjin_amd/libtenjin_host.so, and the C++ time-loop driver used by the tests
 (tests/host/main_loop.cpp) into tests/host/main_loop, the libtorch
 autograd Function over the tangent-linear form (csrc/torch/) into
-tenjin_amd/tenjin_torch.so, and the device-peak kernels (csrc/tj_peaks.hip)
-into tenjin_amd/libtenjin_peaks.so.
+tenjin_amd/tenjin_torch.so, the device-peak kernels (csrc/tj_peaks.hip)
+into tenjin_amd/libtenjin_peaks.so, and the tests' kernel over the library's
+quotients (tests/host/quotients.hip) into tests/host/libquotients.so.
 
 Flags:
   --offload-arch=gfx950            MI355X (CDNA4) only
@@ -90,6 +91,17 @@ def build_peaks(verbose: bool = True) -> str:
     _run([HIPCC] + FLAGS + [src, "-o", PEAKS_LIB + ".tmp"], verbose)
     os.replace(PEAKS_LIB + ".tmp", PEAKS_LIB)
     return PEAKS_LIB
+
+
+QUOTIENTS_LIB = os.path.join(ROOT, "tests", "host", "libquotients.so")
+
+
+def build_quotients(verbose: bool = True) -> str:
+    """The tests' kernel over qdiv and qdivs, with the library's flags."""
+    src = os.path.join(ROOT, "tests", "host", "quotients.hip")
+    _run([HIPCC] + FLAGS + ["-I", CSRC, "-I", INCLUDE, src, "-o", QUOTIENTS_LIB + ".tmp"], verbose)
+    os.replace(QUOTIENTS_LIB + ".tmp", QUOTIENTS_LIB)
+    return QUOTIENTS_LIB
 
 
 TORCH_LIB = os.path.join(HERE, "tenjin_torch.so")

@@ -172,8 +172,9 @@ __device__ __forceinline__ float tdiv(float a, float b) { return a * __builtin_a
 // domain end it is a boundary flux that moves mass and energy in or out.
 __device__ __forceinline__ double tdiv_cr(double a, double b) { return a / b; }
 __device__ __forceinline__ float tdiv_cr(float a, float b) { return a / b; }
-// 1/b by v_rcp_f64 and two Newton steps (a few ulp at worst): the reciprocal
-// that qdiv's quotients and the derivative parts of dual numbers share.
+// 1/b by v_rcp_f64 and two Newton steps, as the compiler's own division refines
+// it (the last step rounds 1/b once): the reciprocal that qdiv's quotients and
+// the derivative parts of dual numbers share.
 __device__ __forceinline__ double drcp(double b) {
     double r = __builtin_amdgcn_rcp(b);
     double e = __builtin_fma(-b, r, 1.0);
@@ -181,22 +182,37 @@ __device__ __forceinline__ double drcp(double b) {
     e = __builtin_fma(-b, r, 1.0);
     return __builtin_fma(r, e, r);
 }
-// a / b correctly rounded, as a / b: the quotient by the reciprocal, corrected
-// by its exact residual (Markstein, IBM J. Res. Dev. 34, 1990), and IEEE's
-// special cases by v_div_fixup_f64.  Written out, so that quotients with one
-// divisor share its reciprocal: 54 cycles a wave for the first and 19 for each
-// further one, against 62 for every a / b, whose sequence also scales both
-// operands by a power of two.  Without the scaling the residual is exact for
-// a = 0 or |a| >= 2^-969 and a divisor in [2^-1021, 2^1021] (and 1e-16 of a
-// smaller a): for divisors that are densities, volume fractions, wave speeds,
-// determinants or material constants, and dividends that are not a wave's
-// vanishing forerunner; the quotients of velocities keep tdiv.
+// a / b by the compiler's own steps (the quotient by the refined reciprocal,
+// corrected by its residual, IEEE's special cases by v_div_fixup_f64) less its
+// scaling of both operands by powers of two, so that quotients with one divisor
+// share its reciprocal: 54 cycles a wave for the first and 19 for each further
+// one, against 62 for every a / b.  The same bits as a / b for zero or
+// non-finite operands, and for a divisor within [2^-500, 2^500) and a dividend
+// within [2^-900, 2^500): densities, wave speeds, material constants, and sums
+// of them.  Outside, the residual of a smaller dividend is not exact (the
+// quotient can be one unit off), and a subnormal divisor or an overflowing
+// quotient gives NaN.  What vanishes ahead of a wave (velocities, shear, strains,
+// mass fractions, a solid's pressure and energy, counted from 0) is divided by
+// tdiv or qdiv0, and by a volume fraction, however small, by tdiv.
 __device__ __forceinline__ double qdiv(double a, double b) {
     const double y = drcp(b);
     const double q = a * y;
     return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
 }
 __device__ __forceinline__ float qdiv(float a, float b) { return tdiv(a, b); }
+// qdiv for every dividend below 2^500, subnormal ones among them: the residual
+// is formed 2^108 times as large, where it is exact for all of them, and scaled
+// back inside the last FMA, which rounds once (a multiplication more: 5 cycles
+// a quotient and 9 a divisor).  A subnormal quotient exactly midway between two
+// numbers may round to either: that takes a divisor that is an even whole
+// number and no power of two.
+__device__ __forceinline__ double qdiv0(double a, double b) {
+    const double y = drcp(b);
+    const double q = a * y;
+    const double r = __builtin_fma(b * -0x1p108, q, a * 0x1p108);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(r, y * 0x1p-108, q), b, a);
+}
+__device__ __forceinline__ float qdiv0(float a, float b) { return tdiv(a, b); }
 // qdiv in the FP64 form, and correctly rounded in FP32 too (see tdiv_cr)
 __device__ __forceinline__ double qdiv_cr(double a, double b) { return qdiv(a, b); }
 __device__ __forceinline__ float qdiv_cr(float a, float b) { return tdiv_cr(a, b); }

@@ -148,6 +148,14 @@ TJ_DUAL_FN Dual<K> qdiv(double a, const Dual<K>& b) {
     for (int t = 0; t < K; ++t) r.d[t] = g * b.d[t];
     return r;
 }
+TJ_DUAL_FN Dual<K> qdiv0(const Dual<K>& a, const Dual<K>& b) {
+    Dual<K> r;
+    r.v = qdiv0(a.v, b.v);
+    const double rb = drcp(b.v);
+#pragma unroll
+    for (int t = 0; t < K; ++t) r.d[t] = __builtin_fma(-r.v, b.d[t], a.d[t]) * rb;
+    return r;
+}
 TJ_DUAL_FN Dual<K> qdiv_cr(const Dual<K>& a, const Dual<K>& b) { return qdiv(a, b); }
 TJ_DUAL_FN Dual<K> operator/(const Dual<K>& a, const Dual<K>& b) { return tdiv(a, b); }
 TJ_DUAL_FN Dual<K> operator/(const Dual<K>& a, double b) { return tdiv(a, b); }

@@ -78,7 +78,7 @@ template <typename R>
 __device__ __forceinline__ R vanleer(R r) {
     if (r <= R(0)) return R(0);
     R num = (r < R(1)) ? R(2) * r : R(2);
-    return qdiv(num, R(1) + r);
+    return tdiv(num, R(1) + r);
 }
 template <typename R>
 __device__ __forceinline__ void muscl1(R um, R uc, R up, R& L, R& Rt) {
@@ -116,7 +116,7 @@ __device__ __forceinline__ R mix_rhob(R lam, R rk, R ra) {
 }
 template <typename R>
 __device__ __forceinline__ void mix_define(const MatT<R>& M, R p, MixV<R>& x) {
-    x.ra = x.rk * (x.lam + (R(1) - x.lam) * qdiv(p - M.pref, p - M.pref2) * qdiv(M.CV2 * M.Gg2, M.CV * M.Gg));
+    x.ra = x.rk * (x.lam + (R(1) - x.lam) * tdiv(p - M.pref, p - M.pref2) * qdiv(M.CV2 * M.Gg2, M.CV * M.Gg));
     x.rb = mix_rhob(x.lam, x.rk, x.ra);
 }
 // mixtureSoundSpeed (equationofstate.cpp:212-226)
@@ -365,7 +365,7 @@ __device__ __forceinline__ unsigned c2p(const Level& lv, const double* al, const
     rho = 0.0;
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = qdiv(ar[m], al[m]);
+        rk[m] = tdiv(ar[m], al[m]);
         rho += ar[m];
     }
     double ke = 0.0;
@@ -381,14 +381,14 @@ __device__ __forceinline__ unsigned c2p(const Level& lv, const double* al, const
         for (int m = 0; m < NM; ++m)
             if (m == lv.mixm) {
                 xm.rk = rk[m];
-                xm.lam = qdiv(arl, ar[m]);
+                xm.lam = tdiv(arl, ar[m]);
             }
         st = root_find<NM>(lv, al, ar, E, ke, xm);
         *x = xm;
     }
     double G, Ent, Pnt;
     eos_sums<NM, double, MX>(lv, al, ar, G, Ent, Pnt, xm);
-    p = qdiv(E - ke - Ent + Pnt, G);
+    p = tdiv(E - ke - Ent + Pnt, G);
     return st;
 }
 

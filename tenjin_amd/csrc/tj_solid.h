@@ -41,7 +41,7 @@ __device__ __forceinline__ void inv3(const R* M, R* Mi) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) Mi[i * 3 + j] = qdiv(cof[j * 3 + i], D);
+        for (int j = 0; j < 3; ++j) Mi[i * 3 + j] = qdiv0(cof[j * 3 + i], D);
 }
 template <typename R>
 __device__ __forceinline__ void mm3(const R* A, const R* B, R* C) {  // C = A B
@@ -441,8 +441,8 @@ template <int NM, typename R>
 __device__ __forceinline__ void c2p_rk_e(const Level& lv, const R* al, const R* ar, const R* are, R* rk, R* e) {
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = qdiv(ar[m], al[m]);
-        e[m] = mat<R>(lv, m).plastic ? qdiv(are[m], ar[m]) : R(0);
+        rk[m] = tdiv(ar[m], al[m]);
+        e[m] = mat<R>(lv, m).plastic ? tdiv(are[m], ar[m]) : R(0);
     }
 }
 
@@ -454,9 +454,9 @@ __device__ __forceinline__ R c2p_s(const Level& lv, const R* al, const R* ar, co
     rho = R(0);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = qdiv(ar[m], al[m]);
+        rk[m] = tdiv(ar[m], al[m]);
         rho += ar[m];
-        e[m] = mat<R>(lv, m).plastic ? qdiv(are[m], ar[m]) : R(0);
+        e[m] = mat<R>(lv, m).plastic ? tdiv(are[m], ar[m]) : R(0);
     }
     const R hj2 = hencky(V, dH);
     R ke = R(0);
@@ -467,7 +467,7 @@ __device__ __forceinline__ R c2p_s(const Level& lv, const R* al, const R* ar, co
     }
     R G, Ent, Pnt;
     eos_sums_s<NM, RW, R>(lv, al, ar, rk, hj2, G, Ent, Pnt);
-    p = qdiv(E - ke - Ent + Pnt, G);
+    p = tdiv(E - ke - Ent + Pnt, G);
     return hj2;
 }
 
@@ -501,7 +501,7 @@ __device__ __forceinline__ void star_s(const Level& lv, const SSt<NM, R>& K, con
     for (int m = 0; m < NM; ++m) {
         T.al[m] = K.al[m];
         T.ar[m] = mult * K.ar[m];
-        T.rk[m] = qdiv(T.ar[m], T.al[m]);
+        T.rk[m] = tdiv(T.ar[m], T.al[m]);
         T.are[m] = mat<R>(lv, m).plastic ? mult * K.are[m] : R(0);
         T.rho += T.ar[m];
     }
@@ -512,7 +512,7 @@ __device__ __forceinline__ void star_s(const Level& lv, const SSt<NM, R>& K, con
 #pragma unroll
         for (int c = 0; c < 3; ++c) T.V[r * 3 + c] = (r == d) ? K.V[r * 3 + c] : mult * K.V[r * 3 + c];
     }
-    T.E = mult * K.rho * (qdiv(K.E, K.rho) + (Ss - K.u[d]) * (Ss - qdiv(K.sig[d], K.rho * (SK - K.u[d]))));
+    T.E = mult * K.rho * (tdiv(K.E, K.rho) + (Ss - K.u[d]) * (Ss - tdiv(K.sig[d], K.rho * (SK - K.u[d]))));
 }
 
 // conservative-variable vector of a state (order of the flux layout):
@@ -648,7 +648,7 @@ __device__ inline void wave5(const Level& lv, const SSt<NM, Rt>& L, const SSt<NM
         const Rt aL = Ls.rho * (Ss - SLT), aR = Rs.rho * (Ss - SRT);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-            sigS[i] = qdiv(Ls.rho * (Ss - SLT) * Rs.rho * (Ss - SRT) * (L.u[i] - R.u[i]) + Ls.rho * (Ss - SLT) * R.sig[i] -
+            sigS[i] = qdiv0(Ls.rho * (Ss - SLT) * Rs.rho * (Ss - SRT) * (L.u[i] - R.u[i]) + Ls.rho * (Ss - SLT) * R.sig[i] -
                                Rs.rho * (Ss - SRT) * L.sig[i],
                            aL - aR);
         Rt uss[NC];
@@ -658,16 +658,16 @@ __device__ inline void wave5(const Level& lv, const SSt<NM, Rt>& L, const SSt<NM
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             if (r == d) continue;
-            uss[2 * NM + r] += qdiv(sigS[r] - K.sig[r], Ss - SKT);
+            uss[2 * NM + r] += qdiv0(sigS[r] - K.sig[r], Ss - SKT);
             ussu[r] = tdiv(uss[2 * NM + r], Ks.rho);
         }
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             if (r == d) continue;
-            uss[2 * NM + 3] += qdiv(ussu[r] * sigS[r] - K.u[r] * K.sig[r], Ss - SKT);
+            uss[2 * NM + 3] += qdiv0(ussu[r] * sigS[r] - K.u[r] * K.sig[r], Ss - SKT);
 #pragma unroll
             for (int c = 0; c < 3; ++c)
-                uss[2 * NM + 4 + r * 3 + c] += qdiv(uss[2 * NM + 4 + d * 3 + c] * (ussu[r] - K.u[r]), Ss - SKT);
+                uss[2 * NM + 4 + r * 3 + c] += qdiv0(uss[2 * NM + 4 + d * 3 + c] * (ussu[r] - K.u[r]), Ss - SKT);
         }
 #pragma unroll
         for (int n = NM; n < NC; ++n) F[n] = f[n] + SK * (uS[n] - uK[n]) + SKT * (uss[n] - uS[n]);
@@ -730,7 +730,7 @@ __device__ inline unsigned plastic_cell(const Level& lv, const R* al, const R* a
     for (int q = 0; q < 9; ++q) {
         const double dl = (q / 3 == q % 3) ? 1.0 : 0.0;
         if (dH[q] != 0.0 && JB == 0.0 && JT != 0.0) st |= 16u;
-        else dH[q] *= qdiv(JT, JB);
+        else dH[q] *= tdiv(JT, JB);
         t1[q] = dl + 0.5 * dH[q];
         t2[q] = dl - 0.5 * dH[q];
     }
@@ -761,7 +761,7 @@ __device__ inline void cleanup_v(const Level& lv, const S* al, S* V) {
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
         const R dl = (q / 3 == q % 3) ? R(1) : R(0);
-        V[q] = (S)qdiv((Sq[q] * norm * tsd) + dl * (ta - tsd), ta);
+        V[q] = (S)qdiv0((Sq[q] * norm * tsd) + dl * (ta - tsd), ta);
     }
 }
 

@@ -425,7 +425,7 @@ __global__ __launch_bounds__(256) void k_tinit_p2c_s(Level lv, DMF<K> U, int shi
 #pragma unroll
         for (int m = 0; m < NM; ++m) ar[m] = P.a[m] * P.r[m];
         eos_sums_s<NM, false, T>(lv, P.a, ar, P.r, U.get(lv.cs[HJ2], i, j, k), G, Ent, Pnt);
-        P.p += qdiv(Pnt, G);
+        P.p += tdiv(Pnt, G);
         U.put(lv.cs[PRESSURE], i, j, k, P.p);
     }
     SSt<NM, T> S;
@@ -768,7 +768,7 @@ __device__ __forceinline__ void tc2p_f(const Level& lv, const Dual<K>* al, const
     rho = T(0.0);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        rk[m] = qdiv(ar[m], al[m]);
+        rk[m] = tdiv(ar[m], al[m]);
         rho += ar[m];
     }
     T ke = T(0.0);
@@ -779,7 +779,7 @@ __device__ __forceinline__ void tc2p_f(const Level& lv, const Dual<K>* al, const
     }
     T G, Ent, Pnt;
     eos_sums<NM, T>(lv, al, ar, G, Ent, Pnt);
-    p = qdiv(E - ke - Ent + Pnt, G);
+    p = tdiv(E - ke - Ent + Pnt, G);
 }
 // getSoundSpeed (sound of tj_fluid.h, no mixture) on dual numbers
 template <int NM, int K>
@@ -980,7 +980,7 @@ __global__ __launch_bounds__(256) void k_tinit_p2c_f(Level lv, DMF<K> U, int shi
 #pragma unroll
         for (int m = 0; m < NM; ++m) ar[m] = P.a[m] * P.r[m];
         eos_sums<NM, T>(lv, P.a, ar, G, Ent, Pnt);
-        P.p += qdiv(Pnt, G);
+        P.p += tdiv(Pnt, G);
         U.put(lv.cs[PRESSURE], i, j, k, P.p);
     }
     FSt<NM, T> S;
