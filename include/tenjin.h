@@ -188,7 +188,10 @@ int tj_compute_dt(tj_ctx* ctx, const tj_mf* U, double* dt_out);
 /* main.cpp:135-143: dt <- min(dt, finalT - t); dt *= 0.2 for step n < 5;
  * operates on the device-resident words (t, n, dt). */
 int tj_driver_dt(tj_ctx* ctx, double final_time);
-/* Sets the device-resident dt (and resets t, n when reset_clock != 0). */
+/* Sets the device-resident dt (and resets t, n when reset_clock != 0).  Waits
+ * for the work queued on the context's stream before the call (its errors are
+ * returned here, and buffers of earlier calls may be used on other streams
+ * afterwards); the new words themselves are queued on the stream. */
 int tj_set_dt(tj_ctx* ctx, double dt, int reset_clock);
 /* Reads the device-resident (t, dt, n). Synchronises. */
 int tj_get_clock(tj_ctx* ctx, double* t, double* dt, int* n);
@@ -211,7 +214,8 @@ int tj_post_step(tj_ctx* ctx, tj_mf* U, unsigned ops);
 int tj_step(tj_ctx* ctx, tj_mf* S, tj_mf* T, int prec);
 
 /* Start of the time loop: t = 0, n = 0, status cleared, and the CFL minimum of
- * the initial state S primed for the first tj_driver_dt. */
+ * the initial state S primed for the first tj_driver_dt.  Waits for the work
+ * queued before the call, as tj_set_dt; its own work is queued. */
 int tj_begin_run(tj_ctx* ctx, const tj_mf* S, double final_time);
 /* nsteps iterations of the loop body of main.cpp:121-191 (tj_driver_dt then
  * tj_step), queued without synchronisation; iterations after the loop test

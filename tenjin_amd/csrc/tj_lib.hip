@@ -601,10 +601,12 @@ int tj_compute_dt(tj_ctx* c, const tj_mf* U, double* dt_out) {
 
 int tj_set_dt(tj_ctx* c, double dt, int reset_clock) {
     if (!c) return TJ_EINVAL;
-    // a launch on the context's stream: a loop driven by the host sets its dt
-    // without waiting for the device (two copies with a wait each before:
-    // 160 x 90 cells 130 -> 74 us a step)
+    // Waits for the work queued before it, as the header states, then queues the
+    // new words as a launch, which a loop driven by the host need not wait for
+    // (it has waited for its dt, so the first wait is empty there; two copies
+    // with a wait each before: 160 x 90 cells 130 -> 74 us a step).
     HIPCHK(c, hipSetDevice(c->device));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     hipLaunchKernelGGL(k_clock_set, dim3(1), dim3(64), 0, c->stream, c->d_clk, dt, reset_clock, c->d_dtpart);
     HIPCHK(c, hipGetLastError());
     return TJ_OK;
