@@ -302,8 +302,10 @@ __device__ __forceinline__ unsigned root_find(const Level& lv, const double* al,
     // trials and about one in the loop take the place of 33.  A y launch of
     // 2048 x 1024 cells: stage 1 488 -> 337 us, stage 2 (two bisections a
     // cell) 846 -> 550, FP32 fluxes 352 -> 236 and 649 -> 464.  A trial's error
-    // is below 16 roundings of the largest terms; the test asks for four times
-    // that.  If it fails, every pass takes its trial.
+    // is below 16 roundings of the largest terms, which for a density above 0
+    // are those at a (with one below 0 the bracket holds v's pole, where they
+    // have no bound); the test asks for four times that.  If it fails, every
+    // pass takes its trial.
     double lo = 0.0, hi = 0.0;
     bool known = false;
     {
@@ -324,7 +326,7 @@ __device__ __forceinline__ unsigned root_find(const Level& lv, const double* al,
         const double r1 = q2 * drcp(t), r2 = t * drcp(q0);
         const double r = (r1 > a && r1 < b) ? r1 : r2;
         const double l = r * (1.0 - 1E-9), h = r * (1.0 + 1E-9);
-        if (l > a && h < b) {
+        if (x.rk > 0.0 && l > a && h < b) {
             const double Ps = (__builtin_fabs(E) + __builtin_fabs(ke) + __builtin_fabs(Ent) + Pm + __builtin_fabs(pal) * va +
                                __builtin_fabs(pbl) * wm) * __builtin_fabs(iG) + __builtin_fabs(M.pref) + __builtin_fabs(M.pref2);
             const double err = 64.0 * 0x1p-53 * Ps * (va * __builtin_fabs(ka) + wm * __builtin_fabs(kb));

@@ -47,14 +47,15 @@ def test_mixture_stage_tiles_match_oracle(nx, ny, thinc):
     assert g.status() == f.status() == o.status()
 
 
-@pytest.mark.parametrize("seed,energy", [(1, 0.0), (2, 0.5), (3, 4.0)])
-def test_bisection_signs_match_oracle(seed, energy):
+@pytest.mark.parametrize("seed,energy,negative", [(1, 0.0, 0), (2, 0.5, 0), (3, 4.0, 0), (4, 0.5, 1), (5, 4.0, 1)])
+def test_bisection_signs_match_oracle(seed, energy, negative):
     """rootFind's known signs: cells whose mass fraction, density, pressure and
     (for energy > 0) total energy are drawn over decades, brackets without a
-    sign change among them, against the oracle's plain bisection, bit for bit."""
+    sign change among them, and (negative) half the cells with a partial density
+    below 0, against the oracle's plain bisection, bit for bit."""
     from oracle.oracle import Oracle
     from tenjin_amd import GpuLevel
-    from tenjin_amd.configs import ALPHA, ALPHARHO, LAMBDA, P, RHO_K, TOTAL_E
+    from tenjin_amd.configs import ALPHA, ALPHARHO, ALPHARHOLAMBDA, LAMBDA, P, RHO_K, TOTAL_E
 
     rng = np.random.default_rng(seed)
     pb = _tube(37, 29, 0)
@@ -72,6 +73,10 @@ def test_bisection_signs_match_oracle(seed, energy):
     s = o.get()
     assert np.array_equal(s[L.comp(ALPHARHO)], g.get_state()[L.comp(ALPHARHO)])
     s[L.comp(TOTAL_E)] *= 10.0 ** (energy * rng.uniform(-1.0, 1.0, shape))
+    if negative:
+        flip = rng.choice([-1.0, 1.0], shape)
+        for c in [L.comp(ALPHARHO, m) for m in range(2)] + [L.comp(ALPHARHOLAMBDA)]:
+            s[c] *= flip
     o.set(s)
     g.set_state(s)
     o.c2p()
