@@ -46,9 +46,9 @@ struct tj_ctx {
     int ncu = 0;  // compute units of the device
     std::map<std::pair<const void*, int>, int> seg_cache;
     bool fuse = false;
-    // two-dimensional fluid levels: each RK stage as the x
-    // and y stage kernels (tj_stage2d.h) over the partially updated state
-    // d_ux, with no flux planes (on by default; off: the flux-plane passes)
+    // two-dimensional fluid levels: each RK stage as the x and y stage kernels
+    // (tj_stage2d.h), in FP64 over the partially updated state d_ux (on by
+    // default; off: the flux-plane passes)
     bool stage2d = true;
     double* d_ux = nullptr;
     // a captured run of loop bodies (tj_graph_capture) and the THINC pass

@@ -979,7 +979,10 @@ static int launch_stage2d(tj_ctx* c, int stage, const MF& in, const MF& base, co
     return TJ_OK;
 }
 
-static bool use_stage2d(const tj_ctx* c) { return c->stage2d && c->d_ux && stage2d_level(c); }
+// The mixed form's stages keep their x fluxes in FP32 planes and need no d_ux.
+static bool use_stage2d(const tj_ctx* c, int prec) {
+    return c->stage2d && stage2d_level(c) && (prec == TJ_PREC_MIXED || c->d_ux);
+}
 
 // One-dimensional fluid levels without a mixture: each RK stage is one launch
 // of k_xstage1d (the x stage completing its cells); with `tail` 1 stage 2 also
@@ -1053,7 +1056,7 @@ int tj_rk_stage(tj_ctx* c, int stage, const tj_mf* Uin, const tj_mf* Ubase, tj_m
     const MF base = stage == 2 ? view(Ubase) : in;
     // the y kernel reads rows of Uin around each tile while other tiles write
     // Uout: an in-place stage (Uout == Uin) takes the flux-plane passes
-    if (use_stage2d(c) && !same_view(view(Uout), in)) return launch_stage2d(c, stage, in, base, view(Uout), 0u, prec);
+    if (use_stage2d(c, prec) && !same_view(view(Uout), in)) return launch_stage2d(c, stage, in, base, view(Uout), 0u, prec);
     if (stage == 1 && use_stage1_solid(c) && !same_view(view(Uout), in)) return launch_stage1_solid(c, in, view(Uout), prec);
     if (use_stage1d(c) && !same_view(view(Uout), in)) return launch_stage1d(c, stage, in, base, view(Uout), 0u, 0, prec);
     const FuseArgs fz{stage, base, view(Uout), 0u};
@@ -1121,7 +1124,7 @@ static int run_step(tj_ctx* c, tj_mf* S, tj_mf* T, int prec, bool next) {
     const MF s = view(S), t = view(T);
     if (same_view(s, t)) { c->err = "step: S and T must be distinct buffers"; return TJ_EINVAL; }
     const bool mixed = prec == TJ_PREC_MIXED;
-    if (use_stage2d(c)) {
+    if (use_stage2d(c, prec)) {
         if ((r = launch_stage2d(c, 1, s, s, t, 0u, prec))) return r;
         if ((r = launch_stage2d(c, 2, t, s, s, step_ops(c), prec))) return r;
         launch_step_end(c, next);
@@ -1695,8 +1698,9 @@ struct Carve {
 };
 
 // The buffers of tj_bind_level for a level, carved from `base` (or only
-// measured, base == null): returns the bytes used.  ux: with the stage
-// kernels' planes (a mixture's stages run on the flux planes without them).
+// measured, base == null): returns the bytes used.  ux: with the FP64 stage
+// kernels' planes (a mixture's stages run on the flux planes without them, and
+// the mixed form has none).
 size_t carve_level(tj_ctx* c, const tj_level_desc* d, unsigned char* base, int prec, bool ux) {
     Carve cv{base};
     Level& lv = c->lv;
@@ -1728,7 +1732,7 @@ size_t carve_level(tj_ctx* c, const tj_level_desc* d, unsigned char* base, int p
             G.p = c->d_fluxf[a];
         }
     }
-    c->d_ux = ux && stage2d_level(c) ? cv.take<double>(lv.ncells * ux_comps(c)) : nullptr;
+    c->d_ux = ux && prec == TJ_PREC_FP64 && stage2d_level(c) ? cv.take<double>(lv.ncells * ux_comps(c)) : nullptr;
     if (d->THINC) {
         const long long pl = lv.ncells * d->nmat;
         c->d_urstar = cv.take<double>(pl);

@@ -86,3 +86,12 @@ def test_run_static_refuses_levels_beyond_its_scratch():
                          ctypes.byref(t), ctypes.byref(n))
     assert rc == TJ_ESCRATCH
     assert np.count_nonzero(a.cpu().numpy()) == 0
+
+
+def test_run_static_mixed_holds_no_fp64_stage_planes():
+    """A mixed level whose scratch fits (61 of 64 MiB) only without the FP64 stage
+    kernels' planes, which the mixed form does not use (12 MiB more)."""
+    from tenjin_amd import TJ_PREC_MIXED, configs
+
+    print("\n[case] tj_run_static: 2D inclusion 608x320, THINC, mixed", flush=True)
+    _run_both(configs.shock_inclusion_2d(nx=608, ny=320, box=32), 4, TJ_PREC_MIXED)
