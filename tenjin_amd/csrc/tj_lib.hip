@@ -794,9 +794,9 @@ static void launch_stage1_solid_t(tj_ctx* c, const MF& in, const MF& out, const 
     const unsigned g = grid1(lv.n[0], T::TC) * grid1(lv.n[1], T::PER - 1) * (unsigned)lv.n[2];
     Timed tm(c, names[mixed][1]);
     if (lv.dim == 2)
-        hipLaunchKernelGGL((k_stage1_s<2, 2, false, R>), dim3(g), dim3(256), 0, c->stream, lv, in, out, F[0], F[2], c->d_clk);
+        hipLaunchKernelGGL((k_stage1_s<2, 2, R>), dim3(g), dim3(256), 0, c->stream, lv, in, out, F[0], F[2], c->d_clk);
     else
-        hipLaunchKernelGGL((k_stage1_s<2, 3, false, R>), dim3(g), dim3(256), 0, c->stream, lv, in, out, F[0], F[2], c->d_clk);
+        hipLaunchKernelGGL((k_stage1_s<2, 3, R>), dim3(g), dim3(256), 0, c->stream, lv, in, out, F[0], F[2], c->d_clk);
 }
 template <typename R, bool MX>
 static void launch_pass_t(tj_ctx* c, const MF& Uin, int d, const FacesT<R>* F, const Hist& h) {
@@ -1036,6 +1036,9 @@ static int launch_stage1d(tj_ctx* c, int stage, const MF& in, const MF& base, co
 // Solid levels of two or three dimensions without Romenskii or Wilkins
 // materials: stage 1 with the y pass and the update in one launch, its output
 // in another buffer than its input (the kernel reads rows around each tile).
+// With those two materials one launch gains next to nothing and loses in 2D: a
+// step in two launches / one takes 7372 / 7325 us on 144^3 in FP64 and 556 /
+// 565 on 512^2 (FP32 fluxes 3857 / 3804 and 353 / 351).
 static bool use_stage1_solid(const tj_ctx* c) { return c->stage2d && c->lv.solid && c->lv.dim >= 2 && !rw_level(c->lv); }
 static int launch_stage1_solid(tj_ctx* c, const MF& in, const MF& out, int prec) {
     if (prec == TJ_PREC_MIXED) launch_stage1_solid_t<float>(c, in, out, c->Ff);

@@ -545,8 +545,9 @@ __global__ __launch_bounds__(256) void k_update_s(Level lv, MF Uin, MF Ub, MF Uo
 // three waves per SIMD alone, two here (144^3 FP64 1363 against 1135 us, FP32
 // fluxes on 203 x 160 x 131 1640 against 1010).  With the z pass in the place
 // of y, whose tile rows lie whole planes apart, stage 1 takes 800 and 890 us
-// against 781 and 826.  DIM: the level's dimensions.
-template <int NM, int DIM, bool RW, typename R>
+// against 781 and 826.  DIM: the level's dimensions.  For levels without
+// Romenskii or Wilkins materials (use_stage1_solid).
+template <int NM, int DIM, typename R>
 __global__ __launch_bounds__(256) void k_stage1_s(Level lv, MF U, MF Uo, FacesT<R> F0, FacesT<R> F2, Clock* clk) {
     using T = STile<NM, R>;
     constexpr int TC = T::TC, FR = T::FR, PER = T::PER - 1;
@@ -562,11 +563,11 @@ __global__ __launch_bounds__(256) void k_stage1_s(Level lv, MF U, MF Uo, FacesT<
     const int tid = threadIdx.x;
     double cand = __builtin_huge_val();
     unsigned st = 0;
-    tile_faces_s<NM, 1, RW, R>(lv, U, lds, i0, c0, k, st);
+    tile_faces_s<NM, 1, false, R>(lv, U, lds, i0, c0, k, st);
     const int cc = tid % TC, f = tid / TC;
     const int i = i0 + cc, j = c0 + 1 + f;
     if (f < PER && i < nx && j < ny) {
-        update_cell_s<NM, 1, RW, R, DIM>(lv, U, U, Uo, i, j, k, clk->dt, 0u, [&](int d, int q, int hi) {
+        update_cell_s<NM, 1, false, R, DIM>(lv, U, U, Uo, i, j, k, clk->dt, 0u, [&](int d, int q, int hi) {
             if (d == 1) return lds[(q * TC + cc) * FR + f + hi];
             return d == 0 ? F0.at(q, i + hi, j, k) : F2.at(q, i, j, k + hi);
         }, cand, st);
