@@ -776,12 +776,14 @@ def main():
 
     def timed(prec):
         """warm-up steps, then exactly args.steps timed steps of the device loop
-        (segment length: --seglen, else the fastest of a few timed on a scratch
-        copy of the level beforehand)"""
+        (segment length where marches run: --seglen, else the fastest of a few
+        timed on a scratch copy of the level beforehand)"""
         fuse = FORMS[args.form]
         seglen = max(args.seglen, 0)
         if fuse == 2 and args.workload in STAGE2D_WORKLOADS:
             tuned[prec] = {"seglen": "unused by the stage kernels"}
+        elif kbytes is SOLID_KERNEL_BYTES:
+            tuned[prec] = {"seglen": "unused by the solid tile passes"}
         elif args.seglen == 0:
             # timed around the middle of the run (at most 250 loop bodies in)
             seglen, trial = autotune.tune_level_seglen(pb, prec, fuse,

@@ -160,10 +160,11 @@ void* tj_stream(tj_ctx* ctx);
  * dx = L/n.  Allocates the scratch (flux planes, THINC history planes).
  * Replaces the set-up of main.cpp:29-95. */
 int tj_bind_level(tj_ctx* ctx, const tj_level_desc* desc);
-/* Tuning: rows per marching segment of the y/z flux passes (seglen > 0
- * fixes it; 0, the default, picks it per pass from the level's shape and the
- * kernel's occupancy so that the segments fill the device's wave slots
- * evenly), and the form of an RK stage:
+/* Tuning: rows per marching segment of a fluid level's y/z flux-plane passes
+ * (seglen > 0 fixes it; 0, the default, picks it per pass from the level's
+ * shape and the kernel's occupancy so that the segments fill the device's wave
+ * slots evenly; solid levels and the stage kernels have no marches), and the
+ * form of an RK stage:
  *   fuse = 2 (default): on two-dimensional fluid levels, the stage kernels --
  *            the x pass with the x part of the update, then the y pass over
  *            LDS tiles with the rest of the update -- and no flux planes; on

@@ -367,10 +367,12 @@ class GpuLevel:
         return s.value
 
     def set_tuning(self, seglen: int = -1, fuse: int = -1):
-        """Rows per marching segment (-1: unchanged) and the form of a stage of a
-        two-dimensional fluid level: 2 the stage kernels (default), 1 flux
-        planes with the update inside the last directional pass, 0 flux planes
-        and a separate update kernel (-1 unchanged)."""
+        """Rows per marching segment of a fluid level's flux-plane passes (-1:
+        unchanged) and the form of a stage: 2 the stage kernels of a
+        two-dimensional fluid level, and a solid level's y pass and stage 1
+        update in one launch (default); 1 flux planes with the update inside a
+        fluid level's last directional pass; 0 flux planes and a separate update
+        kernel (-1 unchanged)."""
         self._chk(self.lib.tj_set_tuning(self.ctx, seglen, fuse), "tj_set_tuning")
 
     def prof_enable(self, on: bool = True):

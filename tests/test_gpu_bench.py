@@ -82,3 +82,15 @@ def test_machine_peaks_are_physical():
         assert isinstance(p[k], float) and 500.0 < p[k] <= 8000.0, (k, p[k])
     assert isinstance(p["fp64_fma_tflops"], float) and 5.0 < p["fp64_fma_tflops"] <= 78.6
     assert isinstance(p["fp32_fma_tflops"], float) and 5.0 < p["fp32_fma_tflops"] <= 157.3
+
+
+def test_bench_tunes_no_segment_length_of_a_solid():
+    """Solid flux passes run in tiles: no segment length to time."""
+    print("\n[case] bench.py --workload plate3d --n3 32 --steps 2 --warmup 1", flush=True)
+    cmd = [sys.executable, os.path.join(ROOT, "bench.py"), "--workload", "plate3d", "--n3", "32", "--box", "16",
+           "--steps", "2", "--warmup", "1", "--no-cpu"]
+    r = subprocess.run(cmd, cwd=ROOT, capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0, r.stderr[-2000:]
+    d = json.loads([l for l in r.stdout.splitlines() if l.startswith("{")][0])
+    tuned = d["config"]["seglen"]
+    assert "fp64" in tuned and all(v == {"seglen": "unused by the solid tile passes"} for v in tuned.values()), tuned
