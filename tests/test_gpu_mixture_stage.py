@@ -21,8 +21,10 @@ def _tube(nx, ny, thinc, box=16):
     return dataclasses.replace(pb, n=(nx, ny, 1), prims=prims)
 
 
-@pytest.mark.parametrize("nx,ny,thinc", [(12, 11, 1), (59, 12, 1), (60, 13, 1), (61, 25, 1), (62, 14, 0), (63, 15, 0),
-                                         (17, 29, 0), (33, 24, 1)])
+CASES = [(12, 11, 1), (59, 12, 1), (60, 13, 1), (61, 25, 1), (62, 14, 0), (63, 15, 0), (17, 29, 0), (33, 24, 1)]
+
+
+@pytest.mark.parametrize("nx,ny,thinc", CASES)
 def test_mixture_stage_tiles_match_oracle(nx, ny, thinc):
     from oracle.oracle import Oracle
     from tenjin_amd import GpuLevel
@@ -45,6 +47,30 @@ def test_mixture_stage_tiles_match_oracle(nx, ny, thinc):
             for c in pb.layout.state_comps():
                 assert np.array_equal(ref[c], got[c]), (step, pb.layout.names[c])
     assert g.status() == f.status() == o.status()
+
+
+@pytest.mark.parametrize("nx,ny,thinc", CASES)
+def test_mixture_stage_tiles_mixed(nx, ny, thinc):
+    """The FP32 instantiations: the stage kernels and the flux-plane passes give
+    the same bits in every component."""
+    from tenjin_amd import TJ_PREC_MIXED, GpuLevel
+
+    pb = _tube(nx, ny, thinc)
+    print(f"\n[case] mixture stage tiles, mixed, {nx} x {ny} thinc {thinc}", flush=True)
+    g, f = GpuLevel(pb), GpuLevel(pb)
+    f.set_tuning(fuse=0)
+    for q in (g, f):
+        q.init_from_prims(pb.prims)
+    for step in range(4):
+        dt = g.compute_dt() * 0.2
+        assert f.compute_dt() * 0.2 == dt
+        for q in (g, f):
+            q.set_dt(dt, reset_clock=1)
+            q.step(TJ_PREC_MIXED)
+        got, planes = g.get_state(), f.get_state()
+        for c in pb.layout.state_comps():
+            assert np.array_equal(got[c], planes[c]), (step, pb.layout.names[c])
+    assert g.status() == f.status()
 
 
 @pytest.mark.parametrize("seed,energy,negative", [(1, 0.0, 0), (2, 0.5, 0), (3, 4.0, 0), (4, 0.5, 1), (5, 4.0, 1)])

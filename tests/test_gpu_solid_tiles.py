@@ -25,9 +25,12 @@ def _plate(n, bc_lo=(0, 0, 0), bc_hi=(0, 0, 0), box=16):
                                prims=np.ascontiguousarray(prims))
 
 
-@pytest.mark.parametrize("n,bc", [
+CASES = [
     ((14, 15), 0), ((15, 14), 1), ((16, 16), 0), ((17, 29), 1), ((30, 30), 0), ((31, 31), 1), ((62, 13), 0),
-    ((63, 32), 1), ((64, 44), 0), ((95, 3), 0), ((3, 46), 1), ((16, 14, 15), 0), ((33, 17, 14), 1), ((5, 31, 16), 0)])
+    ((63, 32), 1), ((64, 44), 0), ((95, 3), 0), ((3, 46), 1), ((16, 14, 15), 0), ((33, 17, 14), 1), ((5, 31, 16), 0)]
+
+
+@pytest.mark.parametrize("n,bc", CASES)
 def test_solid_tiles_match_oracle(n, bc):
     from oracle.oracle import Oracle
     from tenjin_amd import GpuLevel
@@ -50,4 +53,45 @@ def test_solid_tiles_match_oracle(n, bc):
             got = q.get_state()
             for c in pb.layout.state_comps():
                 assert np.array_equal(ref[c], got[c]), (step, pb.layout.names[c])
+    assert g.status() == f.status() == 0
+
+
+# of the largest value of a component's kind: an FP32 flux is off by some 1e-6 of
+# its terms (24-bit operands, a few dozen roundings), of which a step adds a CFL
+# number's part; four steps stay below 1e-5, and a misplaced face is of order 1
+MIXED_TOL = 1e-4
+
+
+@pytest.mark.parametrize("n,bc", CASES)
+def test_solid_tiles_mixed(n, bc):
+    """The FP32 instantiations: both stage forms give the same bits in every
+    component, and all stay by the FP64 state but the phase densities, quotients
+    by volume fractions of 1e-6."""
+    from tenjin_amd import TJ_PREC_MIXED, GpuLevel
+
+    pb = _plate(n, bc_lo=(bc, 0, bc), bc_hi=(0, bc, bc))
+    print(f"\n[case] solid tiles, mixed, {n} bc {bc}", flush=True)
+    d, g, f = GpuLevel(pb), GpuLevel(pb), GpuLevel(pb)
+    f.set_tuning(fuse=0)
+    for q in (d, g, f):
+        q.init_from_prims(pb.prims, pb.shift_pressure)
+    kinds = {}
+    for c in pb.layout.state_comps():
+        kinds.setdefault(pb.layout.names[c].rstrip("0123456789_"), []).append(c)
+    for step in range(4):
+        dt = d.compute_dt() * 0.2
+        d.set_dt(dt, reset_clock=1)
+        d.step()
+        for q in (g, f):
+            q.set_dt(dt, reset_clock=1)
+            q.step(TJ_PREC_MIXED)
+        ref, got, planes = d.get_state(), g.get_state(), f.get_state()
+        for kind, comps in kinds.items():
+            scale = max(np.abs(ref[comps]).max(), 1.0 if kind == "epsilon" else 0.0)
+            if kind == "alphaRhoEpsilon":
+                scale = np.abs(ref[kinds["alphaRho"]]).max()
+            for c in comps:
+                assert np.array_equal(got[c], planes[c]), (step, pb.layout.names[c])
+                err = np.abs(got[c] - ref[c]).max()
+                assert kind == "rho_k" or err <= MIXED_TOL * scale, (step, pb.layout.names[c], err, scale)
     assert g.status() == f.status() == 0
