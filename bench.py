@@ -399,7 +399,7 @@ def bench_ensemble(args):
                    "problems": len(probs), "cells": cells, "precision": "mixed",
                    "launch": f"one hipGraph launch for the whole run ({steps} loop bodies of every problem; capture and "
                              f"instantiation {t_capture:.2f} s, outside the timed region)",
-                   "form": "stage kernels (2D), flux-plane passes (1D)",
+                   "form": "stage kernels (2D), the 1D problems' stages in their x launches",
                    "tile_by_bucket": {str(autotune.BUCKETS[k]): list(BATCH_TILES[v]) for k, v in table.items()},
                    "autotune_s": round(t_tune, 2),
                    "parallelism": "single GPU"},

@@ -195,6 +195,8 @@ void k_b_x12(BTab t1, int q1, int e1, unsigned ops, unsigned b1, BTab t2, int q2
             xstage_body<2, TH, R>(P.lv, STAGE == 1 ? P.S : P.T, P.ux, bhist(P, 0, q2, e2), P.clk, w);
     }
 }
+// No waves are asked for (100 VGPRs in the mixed form's stage 2, four per SIMD):
+// at the single level's six a stage 2 launch takes 244 us in place of 223.
 template <bool TH, int TC, int LPS, int STAGE, typename R>
 __global__ __launch_bounds__(TC * LPS) void k_b_ystage(BTab t, int q, int e, unsigned ops) {
     const long long gb = xcd_block(blockIdx.x, gridDim.x, 2);  // as k_ystage

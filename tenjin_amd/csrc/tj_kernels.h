@@ -840,8 +840,8 @@ __global__ __launch_bounds__(256) void k_sound_dt(Level lv, MF U, Clock* clk) {
 // clamps of main.cpp:121, 135-143.  Re-arms the min word and, with `part`
 // (DT_PARTS words, launched with one wave), first folds the partial slots
 // into it and re-arms them.  With `adv` it first ends the step before
-// (k_clock_advance): between two steps of a run the two are one launch (four
-// steps of three 701 x 389 levels at once 304 -> 300 us each).
+// (k_clock_advance): between two steps of a run the two are one launch instead
+// of two, each of 2 to 5 us between its neighbours on the stream.
 __global__ void k_clock_dt(Clock* clk, double cfl, int driver, unsigned long long* part, int adv) {
     if (blockIdx.x != 0) return;
     if (part) {

@@ -96,13 +96,14 @@ __device__ __forceinline__ void put_face(const R* Fv, Put put) {
 // along D, so a segment of LN lanes gives LN - 1 faces.  The domain's end
 // faces take the image of the edge cell's own state.
 //
-// Bound by VALU issue: some 3500 instructions a face in FP64 (two waves per
-// SIMD), 1900 in FP32 (four).  A march of one wave along D, with the rows in
-// registers, keeps one wave per SIMD in flight and gives a small level few
-// waves: y and z passes of 144^3 in FP64 780 us against 490 here (512^2: 102
-// against 54), of 203 x 160 x 131 in FP32 430 against 285.  Blocks run in XCD
-// order: tiles side by side share the cache lines of rows whose pitch is no
-// multiple of the line (the same FP32 y pass 395 us in round-robin order).
+// Bound by VALU issue: 3100 to 3200 instructions a wave in FP64 (two waves per
+// SIMD; 144^3: x 417 us, y 437, z 442), 1900 in FP32 (four).  A march of one
+// wave along D, with the rows in registers, keeps one wave per SIMD in flight
+// and gives a small level few waves: y and z passes of 144^3 in FP64 780 us
+// against 490 in these tiles (512^2: 102 against 54), both with an IEEE division
+// for every quotient, and of 203 x 160 x 131 in FP32 430 against 285.  Blocks
+// run in XCD order: tiles side by side share the cache lines of rows whose pitch
+// is no multiple of the line (the same FP32 y pass 395 us in round-robin order).
 // The face of a lane: c its lower face along D, PL / PR the reconstructed
 // primitives of its cell, LN lanes to a segment (ld the lane within it).
 // The right state moves up before the left one is built, so two face states
@@ -127,9 +128,9 @@ __device__ __forceinline__ void face_s(const Level& lv, const SPrim<NM, R>& PL, 
     if (face) wave5<NM, RW, R>(lv, Lf, Rf, D, Fv, st);
 }
 
-// x pass: waves of 64 / LN rows by LN lanes along x (144^3 FP64: 555 us with
-// segments of 64, 467 with 32; 203 x 160 x 131 FP32: 340 and 309, and 381 with
-// 16, whose loads fall into four row pieces).
+// x pass: waves of 64 / LN rows by LN lanes along x (144^3 FP64, an IEEE division
+// for every quotient: 555 us with segments of 64, 467 with 32; 203 x 160 x 131
+// FP32: 340 and 309, and 381 with 16, whose loads fall into four row pieces).
 template <int NM, int LN, bool RW, typename R>
 __global__ __launch_bounds__(256) void k_flux_x_s(Level lv, MF U, FacesT<R> F, Clock* clk) {
     if (clk->done) return;
@@ -511,7 +512,7 @@ __device__ __forceinline__ void update_cell_s(const Level& lv, const MF& Uin, co
 }
 
 // Bound by HBM: with 20 flux planes a direction in place of 23, stage 1 of
-// 144^3 FP64 takes 575 us (605), stage 2 715 (760).
+// 144^3 FP64 takes 543 us (23 planes: 605), stage 2 700 (760).
 template <int NM, int STAGE, bool RW, typename T>
 __global__ __launch_bounds__(256) void k_update_s(Level lv, MF Uin, MF Ub, MF Uo, FacesT<T> F0, FacesT<T> F1, FacesT<T> F2,
                                                   Clock* clk, unsigned ops) {
@@ -540,7 +541,7 @@ __global__ __launch_bounds__(256) void k_update_s(Level lv, MF Uin, MF Ub, MF Uo
 // stay in LDS and the update takes the other directions' faces from their
 // planes.  A tile gives 15 faces and completes the 14 cells between them, lanes
 // along x again.  The update alone is bound by HBM and the pass by VALU issue:
-// 144^3 FP64 430 + 575 us as two launches, 790 as one; 512^2 50 + 31 and 69.
+// 144^3 FP64 433 + 543 us as two launches, 839 as one; 512^2 49 + 30 and 69.
 // Stage 2 stays apart: its update has as much arithmetic as a pass and takes
 // three waves per SIMD alone, two here (144^3 FP64 1363 against 1135 us, FP32
 // fluxes on 203 x 160 x 131 1640 against 1010).  With the z pass in the place

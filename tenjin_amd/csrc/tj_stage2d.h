@@ -243,8 +243,8 @@ void k_xstage(Level lv, MF U, UxPlanes Ux, Hist h, Clock* clk) {
 // as k_clock_advance does and re-arms the ticket (no wave waits on another).
 // With `next` it goes on to the next step's dt, as k_clock_dt does: every
 // wave's CFL minimum went into its slot before its ticket, and the slots are
-// read past the caches: two launches a step in place of three (64 steps of
-// three 1000-cell levels at once 421 -> 405 us each).
+// read past the caches: two launches a step in place of three (1000 cells in a
+// graph 18.7 -> 17.9 us a step; about 1 us less at every size up to 1e6 cells).
 template <int NM, bool TH, int STAGE, bool TAIL, typename R = double>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TH && sizeof(R) == 8 ? 4 : 1)))
 void k_xstage1d(Level lv, MF U, MF Ub, MF Uo, Hist h, Clock* clk, unsigned ops, unsigned* ticket, int next) {
@@ -620,9 +620,10 @@ __device__ __forceinline__ void ystage_body(const Level& lv, const MF& U, const 
     if (st) atomicOr(&clk->status, st);
 }
 
-// The mixed form's y kernels take six waves per SIMD (71 VGPRs in stage 2,
-// from 95, no spill): stage 2 0.211 -> 0.202 ms on the 2048 x 1024 level.
-// The FP64 form at five spills about 100 bytes per lane and runs 1.6x slower.
+// The mixed form's y kernels take six waves per SIMD (78 VGPRs in stage 2, 67
+// in stage 1, no spill): stage 2 0.211 -> 0.202 ms on the 2048 x 1024 level when
+// it read the FP64 partial state.  The FP64 form (125) at five spills about 100
+// bytes per lane and runs 1.6x slower.
 // With a mixture (MX) the stages cost 1.8 times less than on the flux planes
 // (512 x 256: 209 against 382 us a step), whose y march has one wave per 64
 // columns and 16 rows: 264 waves there.

@@ -377,11 +377,11 @@ int tj_tangent_create(tj_ctx* c, int ndir, const int* mat, const int* param, int
     tg->par.assign(param, param + ndir);
     tg->ncomp = tj_ncomp(c);
     // groups side by side: as many as fill some four rounds of the device's
-    // waves (the flux kernels run one per SIMD, 1024 together)
+    // waves (the flux kernels run one per SIMD, four to a compute unit)
     const Level& lv = c->lv;
     const int ngroups = (ndir + chunk - 1) / chunk;
     const long long waves = std::max((lv.ncells + 62) / 63, 1LL);
-    tg->rows = (int)std::max(1LL, std::min((long long)ngroups, 4096 / waves));
+    tg->rows = (int)std::max(1LL, std::min((long long)ngroups, 16LL * c->ncu / waves));
     hipError_t e = hipSetDevice(c->device);
     if (e == hipSuccess) e = tg_alloc(tg);
     if (e != hipSuccess && tg->rows > 1) {  // one at a time needs less
